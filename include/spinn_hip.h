@@ -299,6 +299,10 @@ void spinn_hip_tune_streamk(int mode);
  * Change it only between plans: workspace sizes depend on it. No counterpart in the
  * reference. */
 void spinn_hip_tune_winograd_fused(int mode);
+/* The split-bf16 implicit GEMM: mode 1 runs it for every conv it can compute, 0 never,
+ * -1 (default) by the per-shape rule. bm (64 or 128) and split (>= 1) fix its tile height
+ * and K split; 0 leaves them to the rule. */
+void spinn_hip_tune_split_conv(int mode, int bm, int split);
 
 /* Test hook: arrival rounds of the stream-K parts (default 4; < 0 restores
  * it). 0 makes every arrival fail, so the cut tiles stay unwritten and the

@@ -484,6 +484,8 @@ void spinn_hip_tune_streamk_tries(int tries) { force_streamk_tries(tries); }
 
 void spinn_hip_tune_winograd_fused(int mode) { force_winograd_fused(mode); }
 
+void spinn_hip_tune_split_conv(int mode, int bm, int split) { force_split_conv(mode, bm, split); }
+
 const char *spinn_hip_version(void) { return "spinn_amd 0.1 gfx950 fp32-mfma"; }
 
 } // extern "C"

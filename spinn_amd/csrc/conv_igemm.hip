@@ -14,103 +14,11 @@
 // When the tile grid is too small to fill 256 CUs, K is split over blockIdx.z:
 // each split writes raw partial sums to the workspace and a reduction kernel
 // sums them in a fixed order and applies the epilogue (deterministic).
-#include "mfma_core.h"
-#include "spinn_hip_internal.h"
+#include "conv_tile.h"
 #include "streamk.h"
 #include <type_traits>
 
 namespace spinn {
-
-struct ConvKArgs {
-    const float *wpk;  // packed W^T: [group][K][ldw]
-    int64_t wpk_group_stride;
-    int ldw;
-    int M, K;          // per group
-    ConvGeom geom;
-    float *__restrict__ y;
-    const float *__restrict__ bias;
-    const float *__restrict__ res;
-    uint32_t res_bytes; // extent of res (the output's size)
-    int act;
-    int OC, OHW;
-    float *__restrict__ ws; // split-K partials [split][OC][ntot]
-    int k_chunk;       // K per split (multiple of kBK)
-};
-
-// Accumulator start values of a conv output tile: bias + residual when
-// `terms` (their loads then overlap the K loop's prologue instead of arriving
-// as one burst of reads after it, and the epilogue only applies the activation
-// and stores; the sum is the reference's acc + bias + residual in another
-// order, within fp32 rounding), else zero.
-template <class WT>
-__device__ __forceinline__ void conv_acc_start(const ConvKArgs &a, int group, int m0, int n0, int wm0, int wn0,
-                                               int lane, bool terms, f32x16 (&c)[WT::TM][WT::TN]) {
-    if (!terms) {
-        ZeroAcc{}(c);
-        return;
-    }
-    // Unconditional buffer loads: a missing bias or residual is a zero-sized
-    // resource and rows or columns past the edge read at kOOB, all of which
-    // return 0.
-    const int h = lane >> 5;
-    const int l32 = lane & 31;
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(a.bias ? a.bias + group * a.M : a.y, a.bias ? (uint32_t)a.M * 4u : 0u);
-    const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.res ? a.res : a.y, a.res ? a.res_bytes : 0u);
-#pragma unroll
-    for (int j = 0; j < WT::TN; ++j) {
-        const int jcol = n0 + wn0 + j * 32 + l32;
-        const bool col_ok = jcol < a.geom.ntot;
-        const int img = jcol / a.OHW;
-        const int p = jcol - img * a.OHW;
-        const uint32_t ybase = ((uint32_t)img * a.OC + (uint32_t)(group * a.M)) * a.OHW + p;
-#pragma unroll
-        for (int i = 0; i < WT::TM; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                const bool ok = m < a.M;
-                const float bv = buf_f32(rb, ok ? (uint32_t)m * 4u : kOOB);
-                const float rv = buf_f32(rr, ok && col_ok ? (ybase + (uint32_t)m * a.OHW) * 4u : kOOB);
-                c[i][j][r] = bv + rv;
-            }
-    }
-}
-
-// Post-op and store of a finished conv output tile (accumulators already hold
-// bias + residual). Lane owns columns n0 + wn0 + j*32 + lane%32 and rows
-// m0 + wm0 + i*32 + 8*(r/4) + 4*(lane/32) + r%4.
-template <class WT, int AC>
-__device__ __forceinline__ void conv_store(const ConvKArgs &a, int group, int m0, int n0, int wm0, int wn0, int lane,
-                                           const f32x16 (&acc)[WT::TM][WT::TN]) {
-    const int h = lane >> 5;
-    const int l32 = lane & 31;
-    // A tile whose rows all exist (the usual case: OC a multiple of the tile)
-    // stores without a per-element row test.
-    const bool full_m = m0 + WT::WM * WT::WAVES_M <= a.M;
-#pragma unroll
-    for (int j = 0; j < WT::TN; ++j) {
-        const int jcol = n0 + wn0 + j * 32 + l32;
-        if (jcol >= a.geom.ntot) continue;
-        const int img = jcol / a.OHW;
-        const int p = jcol - img * a.OHW;
-        float *yp = a.y + ((int64_t)img * a.OC + (int64_t)group * a.M + m0 + wm0 + 4 * h) * a.OHW + p;
-        if (full_m) {
-#pragma unroll
-            for (int i = 0; i < WT::TM; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    yp[(int64_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * a.OHW] = apply_act_c<AC>(acc[i][j][r]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < WT::TM; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int mo = i * 32 + 8 * (r >> 2) + (r & 3);
-                    if (m0 + wm0 + 4 * h + mo < a.M) yp[(int64_t)mo * a.OHW] = apply_act_c<AC>(acc[i][j][r]);
-                }
-        }
-    }
-}
 
 // AC: the post-op class (act_class), fixed at compile time so the epilogue has no
 // per-element branch on it.
@@ -372,21 +280,7 @@ int launch_conv_tile(const ConvKArgs &a, int groups, int split, hipStream_t st) 
 
 template <int BM, int BN, class BL>
 int launch_conv_sk_tile(const ConvKArgs &a, const SkPlan &sp, int S, void *ws, hipStream_t st) {
-    SkSched s{};
-    s.tiles_m = (a.M + BM - 1) / BM;
-    s.S = S;
-    s.dp_per_xcd = sp.dp_per_xcd;
-    s.R = sp.R;
-    s.scheme = sp.scheme;
-    s.W = sp.W;
-    s.p = sp.p;
-    s.rx = (sp.R + kXcds - 1) / kXcds;
-    s.local = xcd_local_parts() ? 1 : 0;
-    s.epoch = streamk_epoch();
-    s.cnt = (unsigned long long *)ws;
-    s.part = (float *)((char *)ws + sp.cnt_bytes);
-    s.status = device_status_word();
-    s.tries = streamk_tries();
+    const SkSched s = sk_sched(sp, (a.M + BM - 1) / BM, S, ws);
     const dim3 grid(sp.grid);
     if (sp.scheme == kSkSplitWgs) {
         if (act_class(a.act) == 1)
@@ -449,6 +343,14 @@ bool conv_pointwise_vec(const SpinnHipConvDesc *d, const float *x) {
 
 } // namespace
 
+int launch_conv_splitk_reduce(int nsplit, const ConvKArgs &a, hipStream_t st) {
+    const int64_t total = (int64_t)a.OC * a.geom.ntot;
+    const int blocks = (int)std::min<int64_t>((total + 255) / 256, 8192);
+    hipLaunchKernelGGL(conv_splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, a.ws, nsplit, a.OC, a.geom.ntot,
+                       a.OHW, a.bias, a.res, a.act, a.y);
+    return check_launch();
+}
+
 // Floats of the W^T section [group][K][ldw] of the packed weights.
 static int64_t igemm_wt_floats(const SpinnHipConvDesc *d) {
     const int OCg = d->oc / d->group;
@@ -462,10 +364,14 @@ static int64_t igemm_wt_floats(const SpinnHipConvDesc *d) {
 // per 16-byte load, as it does from the raw weights of a 1x1 conv.
 static bool igemm_has_kcopy(const SpinnHipConvDesc *d) { return conv_tap_order(d) && d->kh * d->kw > 1; }
 
-int64_t igemm_packed_floats(const SpinnHipConvDesc *d) {
+// Floats of W^T and, where there is one, the k-contiguous copy, padded to 16 bytes.
+static int64_t igemm_fp32_floats(const SpinnHipConvDesc *d) {
     const int64_t K = (int64_t)(d->c / d->group) * d->kh * d->kw;
-    return igemm_wt_floats(d) + (igemm_has_kcopy(d) ? (int64_t)d->oc * K : 0);
+    return (igemm_wt_floats(d) + (igemm_has_kcopy(d) ? (int64_t)d->oc * K : 0) + 3) / 4 * 4;
 }
+
+// The split planes (split_pack) follow.
+int64_t igemm_packed_floats(const SpinnHipConvDesc *d) { return igemm_fp32_floats(d) + split_packed_floats(d); }
 
 const float *igemm_kcopy(const SpinnHipConvDesc *d, const float *packed) {
     return (packed && igemm_has_kcopy(d)) ? packed + igemm_wt_floats(d) : nullptr;
@@ -479,6 +385,7 @@ int igemm_pack(const SpinnHipConvDesc *d, const float *w, float *packed, hipStre
     hipLaunchKernelGGL(conv_pack_wt_kernel, dim3(blocks), dim3(256), 0, st, w, packed, d->group, OCg,
                        d->c / d->group, d->kh * d->kw, ldw, conv_tap_order(d) ? 1 : 0);
     int rc = check_launch();
+    if (rc == SPINN_HIP_OK) rc = split_pack(d, w, packed + igemm_fp32_floats(d), st);
     if (rc || !igemm_has_kcopy(d)) return rc;
     const int64_t kc = (int64_t)d->oc * (d->c / d->group) * d->kh * d->kw;
     const int kblocks = (int)std::min<int64_t>((kc + 255) / 256, 65535);
@@ -503,7 +410,7 @@ static bool igemm_streamk(const SpinnHipConvDesc *d, const TileChoice &tc, SkPla
     if (d->group != 1 || tc.split > 1) return false;
     const int K = d->c * d->kh * d->kw;
     const int ntot = d->n * d->oh * d->ow;
-    return plan_streamk((d->oc + tc.bm - 1) / tc.bm, (ntot + tc.bn - 1) / tc.bn, (K + kBK - 1) / kBK,
+    return plan_streamk((d->oc + tc.bm - 1) / tc.bm, (ntot + tc.bn - 1) / tc.bn, (K + kBK - 1) / kBK, 4,
                         tc.bm * tc.bn, sp);
 }
 
@@ -517,7 +424,9 @@ static int igemm_wavek(const SpinnHipConvDesc *d) {
 static bool igemm_stem(const SpinnHipConvDesc *d) { return stem_mfma_eligible(d) && !tiles_forced(); }
 
 size_t igemm_workspace_bytes(const SpinnHipConvDesc *d) {
-    if (igemm_stem(d) || igemm_wavek(d)) return 0;
+    if (igemm_stem(d)) return 0;
+    if (split_conv_selected(d)) return split_conv_workspace_bytes(d);
+    if (igemm_wavek(d)) return 0;
     TileChoice tc = igemm_tiles(d);
     SkPlan sp;
     if (igemm_streamk(d, tc, sp)) {
@@ -534,6 +443,8 @@ size_t igemm_workspace_bytes(const SpinnHipConvDesc *d) {
 int igemm_conv(const SpinnHipConvDesc *d, const float *x, const float *w, const float *packed, const float *bias,
                const float *res, float *y, void *ws, size_t ws_bytes, hipStream_t st) {
     if (igemm_stem(d)) return stem_mfma_conv(d, x, packed, bias, res, y, st);
+    if (split_conv_selected(d))
+        return split_conv(d, x, packed + igemm_fp32_floats(d), bias, res, y, ws, ws_bytes, st);
     if (const int ts = igemm_wavek(d)) return wavek_conv(d, ts, x, w, packed, bias, res, y, st);
     ConvKArgs a{};
     const int OCg = d->oc / d->group;
@@ -582,14 +493,7 @@ int igemm_conv(const SpinnHipConvDesc *d, const float *x, const float *w, const 
     else if (d->kh == 1 && d->kw == 1) rc = launch_conv_bl<Gen11BL>(a, tc, d->group, st);
     else rc = launch_conv_bl<GenBL>(a, tc, d->group, st);
     if (rc) return rc;
-    if (tc.split > 1) {
-        const int64_t total = (int64_t)d->oc * a.geom.ntot;
-        const int blocks = (int)std::min<int64_t>((total + 255) / 256, 8192);
-        hipLaunchKernelGGL(conv_splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, (const float *)ws,
-                           tc.split, d->oc, a.geom.ntot, a.OHW, bias, res, d->act, y);
-        rc = check_launch();
-    }
-    return rc;
+    return tc.split > 1 ? launch_conv_splitk_reduce(tc.split, a, st) : rc;
 }
 
 } // namespace spinn

@@ -1,0 +1,210 @@
+// conv_split.hip - where the split-bf16 implicit GEMM (conv_split.h) runs, its weight
+// packing and its launch choice.
+#include "conv_split.h"
+#include <atomic>
+#include <cstdlib>
+
+namespace spinn {
+
+// W [group][OCg][Cg][KH][KW] -> split planes [group][octet][plane][rows_p][8], K in
+// (kh, kw, c) order, each tap's channels padded to octets; one thread per (octet, row).
+__global__ void conv_pack_split_kernel(const float *__restrict__ w, u32x4 *__restrict__ out, int groups, int OCg,
+                                       int Cg, int KHW, int rows_p, int octs) {
+    const int co8 = (Cg + 7) / 8;
+    const int64_t total = (int64_t)groups * octs * rows_p;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
+         e += (int64_t)gridDim.x * blockDim.x) {
+        const int m = (int)(e % rows_p);
+        const int64_t go = e / rows_p;
+        const int o = (int)(go % octs);
+        const int64_t g = go / octs;
+        const int tap = o / co8;
+        const int c0 = (o - tap * co8) * 8;
+        float v[8];
+        for (int i = 0; i < 8; ++i)
+            v[i] = (m < OCg && tap < KHW && c0 + i < Cg) ? w[((g * OCg + m) * Cg + c0 + i) * KHW + tap] : 0.f;
+        u32x4 p[3];
+        split8_weights(v, p[0], p[1], p[2]);
+        u32x4 *dst = out + (go * 3) * rows_p + m;
+        for (int i = 0; i < 3; ++i) dst[(int64_t)i * rows_p] = p[i];
+    }
+}
+
+namespace {
+
+std::atomic<int> g_force_split{-1}, g_force_split_bm{0}, g_force_split_k{0};
+
+struct SplitChoice {
+    int bm, split, chunk, groups_k;
+    bool sk;
+    SkPlan sp;
+};
+
+int split_octs(const SpinnHipConvDesc *d) {
+    const int co8 = (d->c / d->group + 7) / 8;
+    constexpr int q = 4 * kSplitGS;
+    return (d->kh * d->kw * co8 + q - 1) / q * q;
+}
+int split_rows(const SpinnHipConvDesc *d) {
+    return (d->oc / d->group + kSplitRowPad - 1) / kSplitRowPad * kSplitRowPad;
+}
+
+// Tile height, K split and stream-K plan of an eligible conv. A 128-row tile splits each
+// activation half as often as a 64-row one and two workgroups share a CU, so it wins
+// where its grid has a tile per CU (MI355X, us: 512 -> 128@28x28 at batch 32, 392 tiles,
+// 25.4 against 30.1 on 64 rows; 1024 -> 512@14x14 40.5 / 51.8; 3x3 stride 2 128@56x56
+// 62.8 / 79.7), unless M leaves over a fifth of its rows empty. Below that:
+//  * 0.6 to 1 tile per CU and K of 768 or more: 64-row tiles with the remainder cut along
+//    K (3x3 stride 2 256@28x28 at batch 32, 196 tiles: 75.0 against 80.9 on 128 rows
+//    whole, 81.3 on 64 rows whole); a shorter K keeps 128 rows (256 -> 1024@14x14 at
+//    batch 8: 11.3 against 19.8);
+//  * fewer and K of 2048 or more: 128 rows, K split over four tiles' worth of workgroups
+//    (2048 -> 512@7x7 at batch 32: 34.6 against 65.6 unsplit, 44.0 on 64 rows; 3x3 stride
+//    2 512@14x14: 70.1 / 152 / 103);
+//  * else 64 rows, whole.
+// With three or more whole tiles per CU the remainder is cut along K where whole tiles
+// alone are unbalanced (plan_streamk); with fewer the co-resident workgroups even out
+// by themselves (512 -> 128@28x28: 33.8 cut, 25.4 whole).
+SplitChoice split_choice(const SpinnHipConvDesc *d) {
+    SplitChoice c{};
+    const int M = d->oc / d->group;
+    const int ntot = d->n * d->oh * d->ow;
+    const int tiles_n = (ntot + kSplitBN - 1) / kSplitBN;
+    const int64_t cus = device_cu_count();
+    c.groups_k = split_octs(d) / (4 * kSplitGS);
+    c.split = 1;
+    c.chunk = c.groups_k;
+    const int64_t t128 = (int64_t)((M + 127) / 128) * tiles_n * d->group;
+    const bool fills = (M + 127) / 128 * 128 * 4 <= 5 * M;
+    const bool some = 5 * t128 >= 3 * cus && t128 < cus;
+    const bool cut = d->group == 1 && some && c.groups_k >= 12;
+    int split = 1;
+    if (fills && (t128 >= cus || (some && !cut))) {
+        c.bm = 128;
+    } else if (fills && d->group == 1 && !some && 4 * t128 >= cus && c.groups_k >= 32) {
+        c.bm = 128;
+        split = (int)((3 * cus / 2 + t128 - 1) / t128);
+    } else {
+        c.bm = 64;
+    }
+    const bool forced = streamk_forced_on();
+    if (forced) c.bm = 64;
+    if (const int bm = g_force_split_bm.load()) c.bm = bm;
+    if (d->group != 1) return c;
+    if (const int k = g_force_split_k.load()) {
+        split = k;
+    } else if (forced || (cut && c.bm == 64) || (c.bm == 128 && t128 >= 3 * cus)) {
+        c.sk = plan_streamk((M + c.bm - 1) / c.bm, tiles_n, c.groups_k, 1, c.bm * kSplitBN, c.sp);
+        if (c.sk) return c;
+    }
+    split = std::min(split, c.groups_k);
+    if (split > 1) {
+        const int chunk = (c.groups_k + split - 1) / split;
+        c.split = (c.groups_k + chunk - 1) / chunk;
+        c.chunk = c.split > 1 ? chunk : c.groups_k;
+    }
+    return c;
+}
+
+bool split_eligible(const SpinnHipConvDesc *d) {
+    // 16 channels: a slice's octets step at most two taps; the gathers' channel offsets
+    // stay inside the input
+    return d->c / d->group >= 16 && !stem_mfma_eligible(d);
+}
+
+} // namespace
+
+void force_split_conv(int mode, int bm, int split) {
+    g_force_split.store(mode < 0 ? -1 : (mode ? 1 : 0));
+    g_force_split_bm.store(bm == 64 || bm == 128 ? bm : 0);
+    g_force_split_k.store(std::max(split, 0));
+}
+
+bool split_conv_selected(const SpinnHipConvDesc *d) {
+    if (!split_eligible(d) || tiles_forced()) return false;
+    const int f = g_force_split.load();
+    if (f >= 0) return f == 1;
+    const int M = d->oc / d->group;
+    const int K = d->c / d->group * d->kh * d->kw;
+    const int ntot = d->n * d->oh * d->ow;
+    const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((ntot + 63) / 64) * d->group;
+    // Measured against the fp32 MFMA tiles (us): 1x1 with K = 64 gains without a residual
+    // (64 -> 256@56x56 at batch 32: 42.0 -> 34.4) and loses with one (44.1 -> 47.3); grids
+    // under two thirds of a 64 x 64 tile per CU (1024 -> 256@14x14 at batch 8: 15.8 on the
+    // wave-K kernel, 16.8 here) and fewer than 64 rows, half a tile empty, stay there.
+    const bool res = d->act == SPINN_ACT_ADD || d->act == SPINN_ACT_ADD_RELU;
+    return M >= 64 && K >= (res ? 128 : 64) && 3 * tiles64 >= 2 * (int64_t)device_cu_count();
+}
+
+int64_t split_packed_floats(const SpinnHipConvDesc *d) {
+    if (!split_eligible(d)) return 0;
+    return (int64_t)d->group * split_octs(d) * 3 * split_rows(d) * 4;
+}
+
+int split_pack(const SpinnHipConvDesc *d, const float *w, float *packed, hipStream_t st) {
+    if (!split_eligible(d)) return SPINN_HIP_OK;
+    const int64_t total = (int64_t)d->group * split_octs(d) * split_rows(d);
+    const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65535);
+    hipLaunchKernelGGL(conv_pack_split_kernel, dim3(blocks), dim3(256), 0, st, w, (u32x4 *)packed, d->group,
+                       d->oc / d->group, d->c / d->group, d->kh * d->kw, split_rows(d), split_octs(d));
+    return check_launch();
+}
+
+size_t split_conv_workspace_bytes(const SpinnHipConvDesc *d) {
+    const SplitChoice c = split_choice(d);
+    if (c.sk) {
+        // plan time: settle how the parts exchange sums on this device
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess) probe_xcd_local(dev);
+        init_device_status();
+        return c.sp.ws_bytes;
+    }
+    if (c.split <= 1) return 0;
+    return (size_t)c.split * d->oc * ((size_t)d->n * d->oh * d->ow) * sizeof(float);
+}
+
+int split_conv(const SpinnHipConvDesc *d, const float *x, const float *planes, const float *bias, const float *res,
+               float *y, void *ws, size_t ws_bytes, hipStream_t st) {
+    const uint64_t x_bytes = (uint64_t)d->n * d->c * d->h * d->w * sizeof(float);
+    const uint64_t y_bytes = (uint64_t)d->n * d->oc * d->oh * d->ow * sizeof(float);
+    const uint64_t w_bytes = (uint64_t)split_octs(d) * 3 * split_rows(d) * 16;
+    if (x_bytes > kMaxOperandBytes || y_bytes > kMaxOperandBytes || w_bytes > kMaxOperandBytes)
+        return SPINN_HIP_EUNSUPPORTED;
+    const SplitChoice c = split_choice(d);
+    ConvSplitArgs a{};
+    a.t.M = d->oc / d->group;
+    a.t.geom = ConvGeom{x, (uint32_t)x_bytes, d->c, d->h, d->w, d->c / d->group, d->oh, d->ow, d->kh, d->kw,
+                        d->sh, d->sw, d->ph, d->pw, d->n * d->oh * d->ow};
+    a.t.y = y;
+    a.t.bias = bias;
+    a.t.res = res;
+    a.t.res_bytes = (uint32_t)y_bytes;
+    a.t.act = d->act;
+    a.t.OC = d->oc;
+    a.t.OHW = d->oh * d->ow;
+    a.w = SplitPlanes{planes, (uint32_t)w_bytes, split_rows(d), split_octs(d)};
+    a.w_group_stride = (int64_t)w_bytes;
+    a.co8 = (a.t.geom.Cg + 7) / 8;
+    a.groups_k = c.groups_k;
+    a.chunk = c.chunk;
+    SkSched s{};
+    if (c.sk) {
+        if (!ws || ws_bytes < c.sp.ws_bytes || ((uintptr_t)ws & 15u)) return SPINN_HIP_EWORKSPACE;
+        s = sk_sched(c.sp, (a.t.M + c.bm - 1) / c.bm, c.groups_k, ws);
+    } else if (c.split > 1) {
+        if (!ws || ws_bytes < (size_t)c.split * d->oc * (size_t)a.t.geom.ntot * sizeof(float)) return SPINN_HIP_EWORKSPACE;
+        a.t.ws = (float *)ws;
+    }
+    const SkSched *sk = c.sk ? &s : nullptr;
+    const bool pw2 = d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && d->ph == 0 && d->pw == 0 && d->oh == d->h &&
+                     d->ow == d->w && (d->h * d->w) % 2 == 0 && a.t.geom.Cg % 8 == 0 &&
+                     (((uintptr_t)x | (uintptr_t)y | (uintptr_t)res) & 7u) == 0;
+    int rc;
+    if (pw2) rc = launch_conv_split_pw2(a, c.bm, d->group, c.split, sk, c.sp.grid, st);
+    else if (a.t.geom.Cg % 8 == 0) rc = launch_conv_split_gather(a, c.bm, d->group, c.split, sk, c.sp.grid, st);
+    else rc = launch_conv_split_gather_tail(a, c.bm, d->group, c.split, sk, c.sp.grid, st);
+    if (rc || c.split <= 1) return rc;
+    return launch_conv_splitk_reduce(c.split, a.t, st);
+}
+
+} // namespace spinn

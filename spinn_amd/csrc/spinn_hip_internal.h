@@ -93,9 +93,11 @@ struct SkPlan {
     int dp_per_xcd, R, scheme, W, p, grid;
     size_t cnt_bytes, ws_bytes;
 };
-// False when whole tiles are balanced enough (or the split is switched off).
-bool plan_streamk(int tiles_m, int tiles_n, int S, int tile_elems, SkPlan &p);
+// False when whole tiles are balanced enough (or the split is switched off). min_part:
+// the fewest K slices a part done by a whole-tile workgroup may have (64 k).
+bool plan_streamk(int tiles_m, int tiles_n, int S, int min_part, int tile_elems, SkPlan &p);
 void force_streamk(int mode);
+bool streamk_forced_on();
 uint64_t streamk_epoch();
 // Host-visible status word that kernels set when an internal protocol fails
 // (a stream-K arrival that cannot complete): allocated once per process at
@@ -154,6 +156,17 @@ int igemm_pack(const SpinnHipConvDesc *d, const float *w, float *packed, hipStre
 size_t igemm_workspace_bytes(const SpinnHipConvDesc *d);
 int igemm_conv(const SpinnHipConvDesc *d, const float *x, const float *w, const float *packed, const float *bias,
                const float *res, float *y, void *ws, size_t ws_bytes, hipStream_t st);
+
+// split-bf16 implicit GEMM (conv_split.hip): eligible layers' planes follow the fp32 ones
+// in the packed weights; split_conv_selected picks the layers it runs.
+void force_split_conv(int mode, int bm, int split);
+bool split_conv_selected(const SpinnHipConvDesc *d);
+int64_t split_packed_floats(const SpinnHipConvDesc *d);
+int split_pack(const SpinnHipConvDesc *d, const float *w, float *packed, hipStream_t st);
+size_t split_conv_workspace_bytes(const SpinnHipConvDesc *d);
+int split_conv(const SpinnHipConvDesc *d, const float *x, const float *planes, const float *bias, const float *res,
+               float *y, void *ws, size_t ws_bytes, hipStream_t st);
+
 size_t gemm_workspace_bytes(const SpinnHipGemmDesc *d);
 int gemm_run(const SpinnHipGemmDesc *d, const float *A, const float *B, const float *C, float *Y, void *ws,
              size_t ws_bytes, hipStream_t st);

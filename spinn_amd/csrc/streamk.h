@@ -40,6 +40,7 @@
 #include <stdint.h>
 #include "mfma_core.h"
 #include "sk_arrive.h"
+#include "spinn_hip_internal.h"
 
 namespace spinn {
 
@@ -65,6 +66,9 @@ struct SkSched {
     unsigned *status; // host-visible status word: set to 1 when an arrival fails (may be null)
     int tries;       // arrival rounds before giving up (2 always suffice; see sk_arrive.h)
 };
+
+// The launch's schedule over the plan's workspace, with a new epoch.
+SkSched sk_sched(const SkPlan &sp, int tiles_m, int S, void *ws);
 
 // Contiguous share of XCD x in the remaining tiles: [start, start + count).
 __device__ __forceinline__ void sk_xcd_tiles(const SkSched &s, int x, int &start, int &count) {
@@ -192,6 +196,79 @@ __device__ __forceinline__ bool sk_finish_part(const SkSched &s, int nslots, int
         }
     }
     return true;
+}
+
+// The schedule of one workgroup. segment(t, k0, k1, acc) computes K slices [k0, k1) of
+// tile t (starting from the epilogue's terms when k0 == 0) and ends with every wave past
+// its last LDS read of the K loop; store(t, acc) applies the post-op and stores. Segments
+// are unrolled: a loop would keep the second segment's set-up live across the first's K
+// loop.
+template <int SCHEME, int NA, int TILE, class Acc, class Segment, class Store>
+__device__ __forceinline__ void sk_run(const SkSched &s, int tid, int &flag, const Segment &segment,
+                                       const Store &store) {
+    const int id = blockIdx.x;
+    const int nsk = SCHEME == kSkSplitWgs ? kXcds * s.W : 0;
+    const int x = (id < nsk ? id : id - nsk) % kXcds;
+    int xstart, count;
+    sk_xcd_tiles(s, x, xstart, count);
+    const int tile_sk0 = kXcds * s.dp_per_xcd + xstart; // this XCD's first remaining tile
+    if (SCHEME == kSkSplitWgs && id < nsk) {
+        // one range of the XCD's remaining slices
+        const int I = count * s.S;
+        const int Wx = min(s.W, I);
+        const int w = id / kXcds;
+        if (w >= Wx) return; // no slices for this workgroup (uniform exit)
+        const int b = sk_begin(w, I, Wx);
+        const int e = sk_begin(w + 1, I, Wx);
+#pragma unroll
+        for (int seg = 0; seg < 2; ++seg) {
+            const int i = seg == 0 ? b : (b / s.S + 1) * s.S;
+            if (i >= e) break;
+            const int r = i / s.S;
+            const int k0 = i - r * s.S;
+            const int k1 = min(s.S, k0 + (e - i));
+            Acc acc;
+            segment(tile_sk0 + r, k0, k1, acc);
+            if (k0 == 0 && k1 == s.S) {
+                store(tile_sk0 + r, acc);
+            } else {
+                const int w_first = sk_owner(r * s.S, I, Wx);
+                const int nparts = sk_owner((r + 1) * s.S - 1, I, Wx) - w_first + 1;
+                Acc sum;
+                auto slot_of = [&](int q) {
+                    const int wq = w_first + q;
+                    return (x * s.W + wq) * 2 + ((sk_begin(wq, I, Wx) / s.S == r) ? 0 : 1);
+                };
+                if (sk_finish_part<NA, TILE>(s, kXcds * s.W * 2, (x * s.W + w) * 2 + seg, xstart + r, nparts,
+                                             reinterpret_cast<const float *>(&acc), reinterpret_cast<float *>(&sum),
+                                             tid, flag, slot_of))
+                    store(tile_sk0 + r, sum);
+            }
+            __syncthreads(); // the next segment's prologue rewrites the LDS buffers
+        }
+        return;
+    }
+    const int l = (id - nsk) / kXcds; // XCD-local index of this whole-tile workgroup
+    if (SCHEME == kSkPartsInDp && l < count * s.p) {
+        // part j of remaining tile r first
+        const int r = l / s.p;
+        const int j = l - r * s.p;
+        const int k0 = j * s.S / s.p;
+        const int k1 = (j + 1) * s.S / s.p;
+        Acc acc;
+        segment(tile_sk0 + r, k0, k1, acc);
+        Acc sum;
+        const int base = (x * s.rx + r) * s.p;
+        auto slot_of = [&](int q) { return base + q; };
+        if (sk_finish_part<NA, TILE>(s, kXcds * s.rx * s.p, base + j, xstart + r, s.p,
+                                     reinterpret_cast<const float *>(&acc), reinterpret_cast<float *>(&sum), tid, flag,
+                                     slot_of))
+            store(tile_sk0 + r, sum);
+        __syncthreads(); // the whole tile's prologue rewrites the LDS buffers
+    }
+    Acc acc;
+    segment(x * s.dp_per_xcd + l, 0, s.S, acc);
+    store(x * s.dp_per_xcd + l, acc);
 }
 
 } // namespace spinn

@@ -171,7 +171,9 @@ static int env_streamk() {
     return v;
 }
 
-bool plan_streamk(int tiles_m, int tiles_n, int S, int tile_elems, SkPlan &p) {
+bool streamk_forced_on() { return g_force_streamk > 0 || (g_force_streamk < 0 && env_streamk() == 1); }
+
+bool plan_streamk(int tiles_m, int tiles_n, int S, int min_part, int tile_elems, SkPlan &p) {
     const int cus = device_cu_count();
     if (cus % kXcds || tiles_m <= 0 || tiles_n <= 0 || S <= 0) return false;
     const int64_t T = (int64_t)tiles_m * tiles_n;
@@ -203,11 +205,11 @@ bool plan_streamk(int tiles_m, int tiles_n, int S, int tile_elems, SkPlan &p) {
         p.p = 0;
         slots = (size_t)kXcds * p.W * 2;
     } else {
-        // Parts of >= 4 slices, at most one per CU, done by whole-tile
+        // Parts of >= min_part slices, at most one per CU, done by whole-tile
         // workgroups before their own tile.
         p.scheme = kSkPartsInDp;
         p.W = 0;
-        p.p = std::min(std::min(cx / rx, S / 4), kSkMaxParts);
+        p.p = std::min(std::min(cx / rx, S / min_part), kSkMaxParts);
         if (p.p < 2) return false;
         slots = (size_t)kXcds * rx * p.p;
     }
@@ -310,6 +312,25 @@ int take_device_status() {
 
 void force_streamk_tries(int tries) { g_sk_tries.store(tries < 0 ? 4 : tries); }
 int streamk_tries() { return g_sk_tries.load(); }
+
+SkSched sk_sched(const SkPlan &sp, int tiles_m, int S, void *ws) {
+    SkSched s{};
+    s.tiles_m = tiles_m;
+    s.S = S;
+    s.dp_per_xcd = sp.dp_per_xcd;
+    s.R = sp.R;
+    s.scheme = sp.scheme;
+    s.W = sp.W;
+    s.p = sp.p;
+    s.rx = (sp.R + kXcds - 1) / kXcds;
+    s.local = xcd_local_parts() ? 1 : 0;
+    s.epoch = streamk_epoch();
+    s.cnt = (unsigned long long *)ws;
+    s.part = (float *)((char *)ws + sp.cnt_bytes);
+    s.status = device_status_word();
+    s.tries = streamk_tries();
+    return s;
+}
 
 uint64_t streamk_epoch() {
     // 48-bit launch tags, never 0; the start varies between processes.

@@ -1,0 +1,122 @@
+"""Implicit-GEMM convs on the bf16 matrix cores (fp32 operands as three bf16 parts each).
+
+Forced onto shapes at the edges of its tiles and loaders and compared with a float64
+convolution. Bound: an operand's three parts are exact, the products left out stay below
+2^-25 of theirs, and the sum is rounded once per 32 k, so the relative L2 error stays below
+2^-24 (2 + sqrt(K / 32)); twice that is allowed. Inputs that bf16 parts cannot carry
+(infinities, NaN, magnitudes that round to infinity) must give what fp32 arithmetic gives.
+"""
+import ctypes as C
+import math
+import zlib
+
+import numpy as np
+import pytest
+
+from tests.hipops import conv_desc, run_conv
+
+pytestmark = pytest.mark.gpu
+
+# (n, c, h, w, oc, k, stride, pad, group, act)
+SHAPES = [
+    (1, 16, 8, 8, 64, 1, 1, 0, 1, 0),      # smallest K, one column tile, one row tile
+    (2, 64, 7, 10, 65, 1, 1, 0, 1, 5),     # even plane, 2-pixel loads, one row past a tile, residual
+    (3, 72, 7, 7, 130, 1, 1, 0, 1, 3),     # odd plane: gather loads; K no multiple of a slice group
+    (2, 61, 9, 11, 128, 1, 1, 0, 1, 1),    # channels no multiple of 8, ragged columns
+    (1, 16, 13, 13, 96, 3, 2, 1, 1, 1),    # two octets per tap, stride 2
+    (2, 24, 12, 9, 64, 3, 1, 1, 1, 4),     # three octets per tap, residual
+    (1, 19, 10, 10, 80, 5, 2, 2, 1, 0),    # 5x5, channel tail, asymmetric remainder
+    (1, 96, 9, 9, 192, 3, 1, 1, 3, 3),     # grouped
+    (2, 512, 6, 6, 128, 3, 1, 0, 1, 1),    # long K, no padding
+]
+
+
+@pytest.fixture
+def tune(hip):
+    L = hip.lib()
+    yield L.spinn_hip_tune_split_conv
+    L.spinn_hip_tune_split_conv(-1, 0, 0)
+    L.spinn_hip_tune_streamk(-1)
+
+
+def _case(shape):
+    n, c, h, w, oc, k, s, p, g, act = shape
+    rng = np.random.default_rng(zlib.crc32(repr(shape).encode()))
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = (rng.standard_normal((oc, c // g, k, k)) * math.sqrt(2.0 / (c // g * k * k))).astype(np.float32)
+    b = rng.normal(0, 0.1, oc).astype(np.float32)
+    oh, ow = (h + 2 * p - k) // s + 1, (w + 2 * p - k) // s + 1
+    r = rng.standard_normal((n, oc, oh, ow)).astype(np.float32) if act in (4, 5) else None
+    return x, wt, b, r
+
+
+def _exact(torch, shape, x, wt, b, r):
+    n, c, h, w, oc, k, s, p, g, act = shape
+    y = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(),
+                                   torch.from_numpy(b).double(), s, p, 1, g)
+    if r is not None:
+        y = y + torch.from_numpy(r).double()
+    if act in (1, 5):
+        y = torch.where(y < 0, torch.zeros_like(y), y)
+    elif act == 3:
+        y = torch.nn.functional.silu(y)
+    return y.numpy()
+
+
+@pytest.mark.parametrize("bm,split,streamk", [(64, 1, -1), (128, 1, -1), (64, 3, -1), (128, 2, -1), (64, 0, 1)],
+                         ids=["64", "128", "64_ksplit3", "128_ksplit2", "64_streamk"])
+@pytest.mark.parametrize("shape", SHAPES, ids=[repr(s) for s in SHAPES])
+def test_split_conv(hip, torch_gpu, tune, shape, bm, split, streamk):
+    torch = torch_gpu
+    n, c, h, w, oc, k, s, p, g, act = shape
+    if streamk == 1 and g == 1:  # more than a tile per CU, the remainder cut along K
+        tune(1, bm, split)
+        hip.lib().spinn_hip_tune_streamk(streamk)
+        n = 256 * 64 // (((h + 2 * p - k) // s + 1) * ((w + 2 * p - k) // s + 1) * ((oc + 63) // 64))
+        while hip.lib().spinn_hip_conv_workspace_size(C.byref(conv_desc(
+                hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM))) == 0:
+            n += 1
+        shape = (n,) + shape[1:]
+    print(f"[split conv] {shape} bm {bm} split {split} stream-K {streamk}", flush=True)
+    tune(1, bm, split)
+    hip.lib().spinn_hip_tune_streamk(streamk)
+    x, wt, b, r = _case(shape)
+    d = conv_desc(hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch, d, x, wt, b, r)
+    ref = _exact(torch, shape, x, wt, b, r)
+    rel = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    bound = 2 * 2.0 ** -24 * (2 + math.sqrt(c // g * k * k / 32))
+    if act == 3:
+        bound += 1e-6  # the hardware exp2 and reciprocal of SiLU
+    assert rel <= bound, f"relative error {rel:.2e} above {bound:.2e}"
+
+
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[4]], ids=["1x1", "3x3s2"])
+def test_split_conv_special_values(hip, torch_gpu, tune, shape):
+    """Infinities, NaN, values that round to infinity in bf16 and tiny ones, in the input,
+    the weights and the residual."""
+    torch = torch_gpu
+    n, c, h, w, oc, k, s, p, g, act = shape
+    tune(1, 64, 1)
+    x, wt, b, r = _case(shape)
+    x[0, 3, 2, 2], x[0, 5, 4, 7] = np.inf, np.nan
+    x[-1, 2, 5, 5] = 3.4e38
+    x[-1, 7, 0, 0] = 1e-30
+    x[:, 1] *= 1e-3
+    x[0, 1, 6, 5] = -np.inf
+    wt[1] *= 1e-6
+    wt[2, 0, 0, 0], wt[4, 1, 0, 0] = np.inf, 3.4e38
+    if r is not None:
+        r[0, 5, 1, 1] = np.inf
+    d = conv_desc(hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch, d, x, wt, b, r)
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref = _exact(torch, shape, x, wt, b, r)
+    big = np.abs(ref) > 1e37
+    bad = np.argwhere(np.isnan(y) != np.isnan(ref))
+    assert len(bad) == 0, [(tuple(i), y[tuple(i)], ref[tuple(i)]) for i in bad[:8]]
+    inf = np.isinf(ref)
+    assert np.array_equal(y[inf], ref[inf].astype(np.float32))
+    ok = np.isfinite(ref) & ~big
+    assert ok.any() and inf.any()
+    assert np.abs(y[ok] - ref[ok]).max() <= 1e-5 * max(1.0, np.abs(ref[ok]).max())
