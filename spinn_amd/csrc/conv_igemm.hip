@@ -444,7 +444,8 @@ int igemm_conv(const SpinnHipConvDesc *d, const float *x, const float *w, const 
                const float *res, float *y, void *ws, size_t ws_bytes, hipStream_t st) {
     if (igemm_stem(d)) return stem_mfma_conv(d, x, packed, bias, res, y, st);
     if (split_conv_selected(d))
-        return split_conv(d, x, packed + igemm_fp32_floats(d), bias, res, y, ws, ws_bytes, st);
+        return split_conv(d, x, packed, conv_tap_order(d), packed + igemm_fp32_floats(d), bias, res, y, ws, ws_bytes,
+                          st);
     if (const int ts = igemm_wavek(d)) return wavek_conv(d, ts, x, w, packed, bias, res, y, st);
     ConvKArgs a{};
     const int OCg = d->oc / d->group;

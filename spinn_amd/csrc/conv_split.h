@@ -18,6 +18,7 @@ struct ConvSplitArgs {
     int co8;                  // octets per tap
     int groups_k;             // K in groups of slices
     int chunk;                // groups per K split
+    int tap_order;            // t.wpk (fp32 W^T) has K in (kh, kw, c) order, else (c, kh, kw)
 };
 
 template <int CW> struct SplitVec;
@@ -328,25 +329,28 @@ __device__ __forceinline__ void split_conv_segment(const ConvSplitArgs &a, int g
     for (int i = 0; i < T::TM; ++i)
 #pragma unroll
         for (int j = 0; j < T::TN; ++j) acc[i][j] += low[i][j];
-    if (any_nonfinite<T::TM, T::TN>(acc)) {
+    if (out_of_range<T::TM, T::TN>(acc)) {
         split_acc_start<T, RES>(a.t, group, m0, n0, lane, terms, acc);
         const ConvGeom &cg = a.t.geom;
         const __amdgpu_buffer_rsrc_t rx = make_rsrc(cg.x, cg.x_bytes);
+        const float *wt = a.t.wpk + group * a.t.wpk_group_stride;
+        const int taps = cg.KH * cg.KW;
         auto av = [&](int i, int k) {
-            return al.value(w, min(m0 + i * 16 + (lane & 15), w.rows_p - 1), k);
+            const int tap = (k >> 3) / a.co8, c = k - tap * a.co8 * 8;
+            const int m = m0 + i * 16 + (lane & 15);
+            const bool ok = m < a.t.M && tap < taps && c < cg.Cg;
+            return ok ? wt[(int64_t)(a.tap_order ? tap * cg.Cg + c : c * taps + tap) * a.t.ldw + m] : 0.f;
         };
         auto bv = [&](int j, int k) {
             PixelOrigin px;
             px.init(cg, n0 + T::col0(j % T::NQ, lane) + j / T::NQ, group);
-            const int o = k >> 3;
-            const int tap = o / a.co8;
-            const int c = (o - tap * a.co8) * 8 + (k & 7);
+            const int tap = (k >> 3) / a.co8, c = k - tap * a.co8 * 8;
             const int kh = tap / cg.KW;
             const int ih = px.ih0 + kh, iw = px.iw0 + tap - kh * cg.KW;
-            const bool ok = px.valid && kh < cg.KH && c < cg.Cg && (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
+            const bool ok = px.valid && tap < taps && c < cg.Cg && (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
             return buf_f32(rx, ok ? (px.base + (uint32_t)c * (uint32_t)(cg.H * cg.W) + (uint32_t)(ih * cg.W + iw)) * 4u : kOOB);
         };
-        fp32_product<T::TM, T::TN>(g0 * GS * kSplitBK, min(g1 * GS * kSplitBK, w.octs * 8), lane, acc, av, bv);
+        fp32_product<T::TM, T::TN>(g0 * GS * kSplitBK, g1 * GS * kSplitBK, lane, acc, av, bv);
     }
 }
 

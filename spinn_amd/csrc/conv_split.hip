@@ -24,7 +24,7 @@ __global__ void conv_pack_split_kernel(const float *__restrict__ w, u32x4 *__res
         for (int i = 0; i < 8; ++i)
             v[i] = (m < OCg && tap < KHW && c0 + i < Cg) ? w[((g * OCg + m) * Cg + c0 + i) * KHW + tap] : 0.f;
         u32x4 p[3];
-        split8_weights(v, p[0], p[1], p[2]);
+        split8(v, p[0], p[1], p[2]);
         u32x4 *dst = out + (go * 3) * rows_p + m;
         for (int i = 0; i < 3; ++i) dst[(int64_t)i * rows_p] = p[i];
     }
@@ -129,11 +129,12 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     const int ntot = d->n * d->oh * d->ow;
     const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((ntot + 63) / 64) * d->group;
     // Measured against the fp32 MFMA tiles (us): 1x1 with K = 64 gains without a residual
-    // (64 -> 256@56x56 at batch 32: 42.0 -> 34.4) and loses with one (44.1 -> 47.3); grids
+    // (64 -> 256@56x56 at batch 32: 42.0 -> 34.4) and loses with one (44.1 -> 47.3; K = 128,
+    // 128 -> 512@28x28: 36.3 -> 38.8; K = 256, 256 -> 1024@14x14: 33.9 -> 32.4); grids
     // under two thirds of a 64 x 64 tile per CU (1024 -> 256@14x14 at batch 8: 15.8 on the
     // wave-K kernel, 16.8 here) and fewer than 64 rows, half a tile empty, stay there.
     const bool res = d->act == SPINN_ACT_ADD || d->act == SPINN_ACT_ADD_RELU;
-    return M >= 64 && K >= (res ? 128 : 64) && 3 * tiles64 >= 2 * (int64_t)device_cu_count();
+    return M >= 64 && K >= (res ? 256 : 64) && 3 * tiles64 >= 2 * (int64_t)device_cu_count();
 }
 
 int64_t split_packed_floats(const SpinnHipConvDesc *d) {
@@ -163,7 +164,7 @@ size_t split_conv_workspace_bytes(const SpinnHipConvDesc *d) {
     return (size_t)c.split * d->oc * ((size_t)d->n * d->oh * d->ow) * sizeof(float);
 }
 
-int split_conv(const SpinnHipConvDesc *d, const float *x, const float *planes, const float *bias, const float *res,
+int split_conv(const SpinnHipConvDesc *d, const float *x, const float *wt, bool tap_order, const float *planes, const float *bias, const float *res,
                float *y, void *ws, size_t ws_bytes, hipStream_t st) {
     const uint64_t x_bytes = (uint64_t)d->n * d->c * d->h * d->w * sizeof(float);
     const uint64_t y_bytes = (uint64_t)d->n * d->oc * d->oh * d->ow * sizeof(float);
@@ -175,6 +176,11 @@ int split_conv(const SpinnHipConvDesc *d, const float *x, const float *planes, c
     a.t.M = d->oc / d->group;
     a.t.geom = ConvGeom{x, (uint32_t)x_bytes, d->c, d->h, d->w, d->c / d->group, d->oh, d->ow, d->kh, d->kw,
                         d->sh, d->sw, d->ph, d->pw, d->n * d->oh * d->ow};
+    a.t.wpk = wt;
+    a.t.ldw = (a.t.M + 3) / 4 * 4;
+    a.t.K = a.t.geom.Cg * d->kh * d->kw;
+    a.t.wpk_group_stride = (int64_t)a.t.K * a.t.ldw;
+    a.tap_order = tap_order ? 1 : 0;
     a.t.y = y;
     a.t.bias = bias;
     a.t.res = res;

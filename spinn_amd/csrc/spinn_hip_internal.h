@@ -164,8 +164,8 @@ bool split_conv_selected(const SpinnHipConvDesc *d);
 int64_t split_packed_floats(const SpinnHipConvDesc *d);
 int split_pack(const SpinnHipConvDesc *d, const float *w, float *packed, hipStream_t st);
 size_t split_conv_workspace_bytes(const SpinnHipConvDesc *d);
-int split_conv(const SpinnHipConvDesc *d, const float *x, const float *planes, const float *bias, const float *res,
-               float *y, void *ws, size_t ws_bytes, hipStream_t st);
+int split_conv(const SpinnHipConvDesc *d, const float *x, const float *wt, bool tap_order, const float *planes,
+               const float *bias, const float *res, float *y, void *ws, size_t ws_bytes, hipStream_t st);
 
 size_t gemm_workspace_bytes(const SpinnHipGemmDesc *d);
 int gemm_run(const SpinnHipGemmDesc *d, const float *A, const float *B, const float *C, float *Y, void *ws,

@@ -8,11 +8,11 @@
 // 2^-25 of |a*b|, under the rounding of the fp32 sums themselves. Six products at
 // 16x the fp32 MFMA rate leave 2.67x its throughput (157 -> 419 TFLOP/s peak).
 //
-// Values that a sum of three bf16 cannot carry through a product (infinities,
-// NaN, magnitudes that round to infinity) turn every accumulator they reach into
-// NaN or infinity; a wave that finds one after its K loop computes its
-// accumulators again on the fp32 MFMA (recompute), so such inputs give what fp32
-// arithmetic gives.
+// Values that three bf16 parts cannot carry through a product turn every accumulator
+// they reach into NaN or infinity (infinities, NaN, magnitudes that round to infinity)
+// or leave it tiny (below 2^-110 the low parts fall under bf16's least number, 2^-133).
+// A wave that finds such an accumulator after its K loop computes all of its own again
+// on the fp32 MFMA (fp32_product), so these inputs give what fp32 arithmetic gives.
 //
 // A operand (weights): split once when they are packed, laid out as the MFMA
 // reads them, [K/8][3 planes][rows][8 k]: each wave loads its rows' fragments
@@ -76,36 +76,6 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 &hi, u32x4 &mi
     }
 }
 
-// The same for weights, kept exact for every value: an infinity or NaN stays in hi
-// alone, and a finite value whose bf16 would round to infinity takes the largest
-// finite one, so hi + mid + lo gives the fp32 value back.
-__device__ __forceinline__ void split8_weights(const float (&v)[8], u32x4 &hi, u32x4 &mid, u32x4 &lo) {
-    float f[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = v[i];
-    split8(f, hi, mid, lo);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t u = __builtin_bit_cast(uint32_t, v[i]);
-        if ((u & 0x7f800000u) == 0x7f800000u || (u & 0x7fffffffu) >= 0x7f7f8000u) {
-            uint32_t h = u >> 16, m = 0, l = 0;
-            if ((u & 0x7f800000u) == 0x7f800000u) {
-                if (u & 0x007fffffu) h |= 0x40u; // a NaN whose payload lies in the low half stays NaN
-            } else {
-                uint32_t hp, mp, lp;
-                split2(v[i] - __builtin_bit_cast(float, h << 16), 0.f, hp, mp, lp);
-                m = hp & 0xffffu;
-                l = mp & 0xffffu;
-            }
-            const int sh = (i & 1) * 16;
-            const uint32_t keep = ~(0xffffu << sh);
-            hi[i / 2] = (hi[i / 2] & keep) | (h << sh);
-            mid[i / 2] = (mid[i / 2] & keep) | (m << sh);
-            lo[i / 2] = (lo[i / 2] & keep) | (l << sh);
-        }
-    }
-}
-
 // LDS buffer of one group of slices of the split B operand: [octet][plane][64 + 2] runs
 // of 16 bytes.
 constexpr int kSplitRow = kSplitBN + 2;
@@ -152,15 +122,6 @@ struct PlanesA {
                 a[i][p] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
                                                          rsrc, (int)voff[i], (int)(s + p * plane_bytes), 0));
     }
-    // One fp32 weight back from its parts (exact).
-    __device__ __forceinline__ float value(const SplitPlanes &p, int row, int k) const {
-        const uint16_t *q = (const uint16_t *)p.base + ((int64_t)(k >> 3) * 3 * p.rows_p + row) * 8 + (k & 7);
-        float v[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            v[i] = __builtin_bit_cast(float, (uint32_t)q[(int64_t)i * p.rows_p * 8] << 16);
-        return (v[0] + v[1]) + v[2];
-    }
 };
 
 template <int T>
@@ -190,17 +151,23 @@ __device__ __forceinline__ void split_mfma(const bf16x8 (&a)[TM][3], const bf16x
         }
 }
 
-// True when any accumulator of the wave is infinite or NaN.
+// True when any accumulator of the wave is infinite, NaN, or nonzero below 2^-80, which
+// sums of ordinary values do not cancel down to (their residue is 2^-24 of a term).
 template <int TM, int TN>
-__device__ __forceinline__ bool any_nonfinite(const f32x4 (&acc)[TM][TN]) {
-    float s = 0.f; // v * 0 is 0 for finite v and NaN otherwise; a NaN survives the sums
+__device__ __forceinline__ bool out_of_range(const f32x4 (&acc)[TM][TN]) {
+    constexpr uint32_t kTiny = (127u - 80u) << 23;
+    float s = 0.f;         // v * 0 is 0 for finite v and NaN otherwise; a NaN survives the sums
+    uint32_t low = ~0u;    // least |v| - 1 as bits: zero wraps to the largest
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s += acc[i][j][r] * 0.f;
-    return __any(s != s);
+            for (int r = 0; r < 4; ++r) {
+                s += acc[i][j][r] * 0.f;
+                low = min(low, (__builtin_bit_cast(uint32_t, acc[i][j][r]) & 0x7fffffffu) - 1u);
+            }
+    return __any(s != s || low < kTiny);
 }
 
 // Accumulators of one wave again in fp32: av(i, k) and bv(j, k) give the lane's

@@ -120,3 +120,22 @@ def test_split_conv_special_values(hip, torch_gpu, tune, shape):
     ok = np.isfinite(ref) & ~big
     assert ok.any() and inf.any()
     assert np.abs(y[ok] - ref[ok]).max() <= 1e-5 * max(1.0, np.abs(ref[ok]).max())
+
+
+@pytest.mark.parametrize("sx,sw", [(1e-36, 1.0), (1.0, 1e-36), (1e-20, 1e-16), (1e30, 1e5)])
+@pytest.mark.parametrize("shape", [(2, 64, 7, 10, 65, 1, 1, 0, 1, 0), (1, 19, 10, 10, 80, 3, 1, 1, 1, 0)],
+                         ids=["1x1", "3x3_tail"])
+def test_split_conv_scales(hip, torch_gpu, tune, shape, sx, sw):
+    """Magnitudes whose low parts lie under bf16's least number, and large ones: the error
+    stays relative to the result."""
+    n, c, h, w, oc, k, s, p, g, act = shape
+    tune(1, 64, 1)
+    x, wt, _, _ = _case(shape)
+    x, wt = (x * np.float32(sx)).astype(np.float32), (wt * np.float32(sw)).astype(np.float32)
+    d = conv_desc(hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch_gpu, d, x, wt)
+    ref = _exact(torch_gpu, shape, x, wt, np.zeros(oc, np.float32), None)
+    scale = ref.std()
+    rel = np.linalg.norm(y / scale - ref / scale) / np.linalg.norm(ref / scale)
+    # fp32 sums of K terms in two-term steps on the fp32 path
+    assert rel <= 2 * 2.0 ** -24 * (2 + math.sqrt(c * k * k / 2))
