@@ -75,42 +75,65 @@ __global__ __launch_bounds__(256) void reduce_max_short_kernel(const float *__re
     }
 }
 
-// Short rows of a multiple of 16 floats (a detector's 80 class scores): four
-// lanes per row, each scanning a contiguous quarter in float4 steps with the
-// reference's rule, then the quarters combined in index order (a later
-// quarter's maximum replaces the running one only when strictly greater):
-// for NaN-free rows the first maximal element, as the single scan finds it,
-// with four times the threads (8400 rows at batch 1: 132 workgroups, not 33).
+// The same over rows of a multiple of 16 floats (16-byte aligned): four lanes per row.
+// The result is the row's first maximal element as quarters of the row find it, each
+// scanned in index order from its first element under `v > best`, a later quarter's
+// replacing the running one only when strictly greater. Which element comes first only
+// shows where equal elements differ in their bits (zeros of either sign) or where a NaN
+// is about, so a row is first read with the four lanes on neighbouring float4s, 64
+// contiguous bytes a step instead of four runs a quarter row apart, every load issued
+// before the first comparison; a row whose maximum is zero or that holds a NaN is then
+// scanned by quarters. 134400 rows of 80 (43 MB,
+// memory bound): 15.4 -> 7.5 us of the detector's post-processing (71.0 -> 63.1 us).
+template <int NV> // float4s per lane
 __global__ __launch_bounds__(256) void reduce_max_short4_kernel(const float *__restrict__ x, float *__restrict__ y,
-                                                                int64_t rows, int block) {
+                                                                int64_t rows) {
+    constexpr int block = NV * 16;
     const int64_t total = rows * 4;
-    const int len = block >> 2; // a multiple of 4
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < total; base += (int64_t)gridDim.x * blockDim.x) {
         const int64_t t = base + threadIdx.x; // uniform trip count: every lane reaches the shuffles
         const bool live = t < total;
-        const int64_t row = t >> 2;
         const int q = (int)(t & 3);
-        float best = 0.f;
-        if (live) {
-            const float *xr = x + row * block + (int64_t)q * len;
-            best = xr[0];
-            for (int j = 0; j < len; j += 4) {
-                const float4 v = *reinterpret_cast<const float4 *>(xr + j);
-                if (v.x > best) best = v.x;
-                if (v.y > best) best = v.y;
-                if (v.z > best) best = v.z;
-                if (v.w > best) best = v.w;
+        const float *xr = x + (live ? t >> 2 : rows - 1) * block;
+        float4 v[NV];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[j] = *reinterpret_cast<const float4 *>(xr + (j * 4 + q) * 4);
+        float best = v[0].x;
+        float nan = 0.f; // NaN once the lane has seen one (infinities aside: inf * 0 is NaN too)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            best = fmaxf(fmaxf(fmaxf(best, v[j].x), fmaxf(v[j].y, v[j].z)), v[j].w);
+            nan += v[j].x * 0.f + v[j].y * 0.f + v[j].z * 0.f + v[j].w * 0.f;
+        }
+#pragma unroll
+        for (int off = 1; off <= 2; off <<= 1) {
+            best = fmaxf(best, __shfl_xor(best, off, 64));
+            nan += __shfl_xor(nan, off, 64);
+        }
+        if (best == 0.f || nan != nan) { // the same for a row's four lanes
+            const float *xq = xr + q * (block / 4);
+            best = xq[0];
+            for (int j = 0; j < block / 4; ++j)
+                if (xq[j] > best) best = xq[j];
+            const int lead = (int)(threadIdx.x & 63) & ~3;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const float b = __shfl(best, lead + p, 64);
+                if (p == 0) nan = b;
+                else if (b > nan) nan = b;
             }
+            best = nan;
         }
-        const int lead = (int)(threadIdx.x & 63) & ~3;
-        const float b1 = __shfl(best, lead + 1, 64), b2 = __shfl(best, lead + 2, 64), b3 = __shfl(best, lead + 3, 64);
-        if (live && q == 0) {
-            float m = best;
-            if (b1 > m) m = b1;
-            if (b2 > m) m = b2;
-            if (b3 > m) m = b3;
-            y[row] = m;
-        }
+        if (live && q == 0) y[t >> 2] = best;
+    }
+}
+
+template <int NV>
+void launch_reduce_max_short4(int nv, const float *x, float *y, int64_t rows, hipStream_t st) {
+    if constexpr (NV > 0) {
+        if (nv != NV) return launch_reduce_max_short4<NV - 1>(nv, x, y, rows, st);
+        const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>((rows * 4 + 255) / 256, 65536)));
+        hipLaunchKernelGGL(reduce_max_short4_kernel<NV>, grid, dim3(256), 0, st, x, y, rows);
     }
 }
 
@@ -587,8 +610,7 @@ int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n 
 
 int reduce_max_rows(int64_t rows, int64_t block, const float *x, float *y, hipStream_t st) {
     if (block <= 256 && block % 16 == 0 && ((uintptr_t)x & 15u) == 0 && rows <= INT64_MAX / 4) {
-        const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>((rows * 4 + 255) / 256, 65536)));
-        hipLaunchKernelGGL(reduce_max_short4_kernel, grid, dim3(256), 0, st, x, y, rows, (int)block);
+        launch_reduce_max_short4<16>((int)block / 16, x, y, rows, st);
         return check_launch();
     }
     if (block <= 256) {
