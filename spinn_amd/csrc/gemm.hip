@@ -29,7 +29,12 @@ struct GemmKArgs {
     int k_chunk;
 };
 
-template <int BM, int BN, int BK, class ALoader, class BLoader, bool SPLIT>
+// SETS: accumulator sets of the K loop. One chain over a K of some hundreds rounds more
+// than the wave-K kernel's eight; grids of at most two 64 x 64 tiles per CU, which leave
+// the registers free, take four (the detector's attention at batch 16, two of whose
+// products these are: 4.3e-7 -> 2.9e-7 against 64 bits, 29.9 -> 30.7 us; 36.3 us with the
+// second product on the wave-K kernel).
+template <int BM, int BN, int BK, class ALoader, class BLoader, bool SPLIT, int SETS>
 __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmKArgs a) {
     using WT = WaveTiling<BM, BN>;
     constexpr int SA = LdsPad<BM>::stride;
@@ -69,7 +74,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmKArgs a) {
 
     f32x16 acc[WT::TM][WT::TN];
     const int nslices = (k_end - k_begin + BK - 1) / BK;
-    gemm_mainloop<BM, BN, BK, kStages>(al, bl, As, Bs, acc, k_begin, nslices, tid, lane, wm0, wn0, ZeroAcc{});
+    if constexpr (SETS > 1) {
+        AccSets<SETS, WT::TM, WT::TN> sets;
+        gemm_mainloop<BM, BN, BK, kStages>(al, bl, As, Bs, sets, k_begin, nslices, tid, lane, wm0, wn0, ZeroAcc{});
+        sets.sum(acc);
+    } else {
+        gemm_mainloop<BM, BN, BK, kStages>(al, bl, As, Bs, acc, k_begin, nslices, tid, lane, wm0, wn0, ZeroAcc{});
+    }
 
     // Epilogue: C values of a column block are loaded before any store.
     const int h = lane >> 5;
@@ -228,10 +239,17 @@ namespace {
 template <int BM, int BN, class AL, class BL>
 int launch_gemm_tile(const GemmKArgs &a, int batch, int split, hipStream_t st) {
     dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM, split > 1 ? split : batch);
-    if (split > 1)
-        hipLaunchKernelGGL((gemm_kernel<BM, BN, kBK, AL, BL, true>), grid, dim3(kThreads), 0, st, a);
-    else
-        hipLaunchKernelGGL((gemm_kernel<BM, BN, kBK, AL, BL, false>), grid, dim3(kThreads), 0, st, a);
+    if (split > 1) {
+        hipLaunchKernelGGL((gemm_kernel<BM, BN, kBK, AL, BL, true, 1>), grid, dim3(kThreads), 0, st, a);
+        return check_launch();
+    }
+    if constexpr (BM == 64 && BN == 64) {
+        if ((int64_t)grid.x * grid.y * grid.z <= 2 * (int64_t)device_cu_count()) {
+            hipLaunchKernelGGL((gemm_kernel<BM, BN, kBK, AL, BL, false, 4>), grid, dim3(kThreads), 0, st, a);
+            return check_launch();
+        }
+    }
+    hipLaunchKernelGGL((gemm_kernel<BM, BN, kBK, AL, BL, false, 1>), grid, dim3(kThreads), 0, st, a);
     return check_launch();
 }
 

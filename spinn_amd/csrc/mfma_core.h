@@ -448,17 +448,38 @@ __device__ __forceinline__ void load_fragments(const float *__restrict__ As, con
     }
 }
 
-template <int BM, int BN, int BK, int Q0, int Q1>
+// The accumulators of a wave as the K loop sees them: one set, or N sets taken in turn by
+// consecutive K steps and added at the end (sum()), which rounds each running sum N times
+// less often.
+template <int N, int TM, int TN>
+struct AccSets {
+    f32x16 v[N][TM][TN];
+    __device__ __forceinline__ void sum(f32x16 (&out)[TM][TN]) const {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                out[i][j] = v[0][i][j];
+#pragma unroll
+                for (int n = 1; n < N; ++n) out[i][j] += v[n][i][j];
+            }
+    }
+};
+template <int TM, int TN>
+__device__ __forceinline__ f32x16 &acc_at(f32x16 (&acc)[TM][TN], int, int i, int j) { return acc[i][j]; }
+template <int N, int TM, int TN>
+__device__ __forceinline__ f32x16 &acc_at(AccSets<N, TM, TN> &acc, int q, int i, int j) { return acc.v[q % N][i][j]; }
+
+template <int BM, int BN, int BK, int Q0, int Q1, class Acc>
 __device__ __forceinline__ void mfma_steps(const float (&a)[BK / 2][WaveTiling<BM, BN>::TM],
-                                           const float (&b)[BK / 2][WaveTiling<BM, BN>::TN],
-                                           f32x16 (&acc)[WaveTiling<BM, BN>::TM][WaveTiling<BM, BN>::TN]) {
+                                           const float (&b)[BK / 2][WaveTiling<BM, BN>::TN], Acc &acc) {
 #pragma unroll
     for (int q = Q0; q < Q1; ++q)
 #pragma unroll
         for (int i = 0; i < WaveTiling<BM, BN>::TM; ++i)
 #pragma unroll
             for (int j = 0; j < WaveTiling<BM, BN>::TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][i], b[q][j], acc[i][j], 0, 0, 0);
+                acc_at(acc, q, i, j) = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][i], b[q][j], acc_at(acc, q, i, j), 0, 0, 0);
 }
 
 // One pipelined slice: MFMAs of slice s (from LDS buffer `cur`), with the
@@ -467,10 +488,9 @@ __device__ __forceinline__ void mfma_steps(const float (&a)[BK / 2][WaveTiling<B
 // Both happen unconditionally: a fetch past the end of K reads through the
 // operand's bounded buffer descriptor (zeros, or data the loop never
 // consumes), so no branch hides the load count from the wait-count logic.
-template <int BM, int BN, int BK, class AL, class BL>
+template <int BM, int BN, int BK, class AL, class BL, class Acc>
 __device__ __forceinline__ void pipelined_slice(AL &al, BL &bl, const float *As_cur, const float *Bs_cur,
-                                                float *As_nxt, float *Bs_nxt,
-                                                f32x16 (&acc)[WaveTiling<BM, BN>::TM][WaveTiling<BM, BN>::TN],
+                                                float *As_nxt, float *Bs_nxt, Acc &acc,
                                                 int k_fetch, int tid, int lane, int wm0, int wn0) {
     float a[BK / 2][WaveTiling<BM, BN>::TM], b[BK / 2][WaveTiling<BM, BN>::TN];
     load_fragments<BM, BN, BK>(As_cur, Bs_cur, a, b, wm0, wn0, lane);
@@ -500,12 +520,10 @@ __device__ __forceinline__ void pipelined_slice(AL &al, BL &bl, const float *As_
 // stage is a copy of them. `init(acc)` sets the accumulators' start values;
 // it runs right after the first slice's loads are issued, so loads it makes
 // (a fused epilogue's bias and residual) overlap the prologue.
-template <int BM, int BN, int BK, int NS, class AL, class BL, class Init>
+template <int BM, int BN, int BK, int NS, class AL, class BL, class Init, class Acc>
 __device__ __forceinline__ void gemm_mainloop(const AL &al_init, const BL &bl_init,
                                               float (*As)[BK * LdsPad<BM>::stride],
-                                              float (*Bs)[BK * LdsPad<BN>::stride],
-                                              f32x16 (&acc)[WaveTiling<BM, BN>::TM][WaveTiling<BM, BN>::TN],
-                                              int k_begin, int nslices, int tid, int lane, int wm0, int wn0,
+                                              float (*Bs)[BK * LdsPad<BN>::stride], Acc &acc, int k_begin, int nslices, int tid, int lane, int wm0, int wn0,
                                               const Init &init) {
     static_assert(NS >= 2 && NS % 2 == 0, "the LDS buffer of a slice is its parity: NS must be even");
     if (nslices <= 0) {
