@@ -130,11 +130,15 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((ntot + 63) / 64) * d->group;
     // Measured against the fp32 MFMA tiles (us): 1x1 with K = 64 gains without a residual
     // (64 -> 256@56x56 at batch 32: 42.0 -> 34.4) and loses with one (44.1 -> 47.3; K = 128,
-    // 128 -> 512@28x28: 36.3 -> 38.8; K = 256, 256 -> 1024@14x14: 33.9 -> 32.4); grids
-    // under two thirds of a 64 x 64 tile per CU (1024 -> 256@14x14 at batch 8: 15.8 on the
-    // wave-K kernel, 16.8 here) and fewer than 64 rows, half a tile empty, stay there.
+    // 128 -> 512@28x28: 36.3 -> 38.8; K = 256, 256 -> 1024@14x14: 33.9 -> 32.4). Grids of
+    // two thirds to one 64 x 64 tile per CU gain from K = 256 (384 -> 256@13x13 at batch 16:
+    // 13.4 -> 12.3; K = 128, 128@80x80 at batch 1: 6.06 and 6.09) and smaller ones lose
+    // (1024 -> 256@14x14 at batch 8: 15.8 on the wave-K kernel, 16.8 here), as do rows that
+    // leave over a quarter of the tiles empty (80@80x80 at batch 1: 5.2 -> 5.9).
     const bool res = d->act == SPINN_ACT_ADD || d->act == SPINN_ACT_ADD_RELU;
-    return M >= 64 && K >= (res ? 256 : 64) && 3 * tiles64 >= 2 * (int64_t)device_cu_count();
+    const int64_t cus = device_cu_count();
+    if ((M + 63) / 64 * 64 * 3 > 4 * M || K < (res ? 256 : 64)) return false;
+    return tiles64 >= cus || (3 * tiles64 >= 2 * cus && K >= 256);
 }
 
 int64_t split_packed_floats(const SpinnHipConvDesc *d) {

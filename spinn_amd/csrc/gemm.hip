@@ -30,8 +30,9 @@ struct GemmKArgs {
 };
 
 // SETS: accumulator sets of the K loop. One chain over a K of some hundreds rounds more
-// than the wave-K kernel's eight; grids of at most two 64 x 64 tiles per CU, which leave
-// the registers free, take four (the detector's attention at batch 16, two of whose
+// than the wave-K kernel's eight; the grids that take 64 x 64 tiles in its place (under one
+// per CU, K of 128..576) use four, others one (2611 x 421 x 93, 287 tiles: 12.6 us with one
+// set, 14.0 with four) (the detector's attention at batch 16, two of whose
 // products these are: 4.3e-7 -> 2.9e-7 against 64 bits, 29.9 -> 30.7 us; 36.3 us with the
 // second product on the wave-K kernel).
 template <int BM, int BN, int BK, class ALoader, class BLoader, bool SPLIT, int SETS>
@@ -244,7 +245,7 @@ int launch_gemm_tile(const GemmKArgs &a, int batch, int split, hipStream_t st) {
         return check_launch();
     }
     if constexpr (BM == 64 && BN == 64) {
-        if ((int64_t)grid.x * grid.y * grid.z <= 2 * (int64_t)device_cu_count()) {
+        if ((int64_t)grid.x * grid.y * grid.z < device_cu_count() && a.K >= 128 && a.K <= 576) {
             hipLaunchKernelGGL((gemm_kernel<BM, BN, kBK, AL, BL, false, 4>), grid, dim3(kThreads), 0, st, a);
             return check_launch();
         }

@@ -22,8 +22,8 @@ GEMMS = [
     (64, 400, 400, 0, 1, 32),    # 224 64 x 64 tiles
     (65, 129, 576, 0, 0, 22),    # ragged 64 x 64 tiles
     (500, 1000, 130, 1, 1, 1),   # 128 of them
-    (2048, 1000, 97, 0, 1, 1),   # 512: the most with four accumulator sets
-    (2048, 1025, 97, 0, 1, 1),   # 544: one set
+    (960, 1088, 128, 0, 1, 1),   # 255: the most with four accumulator sets
+    (1024, 1024, 128, 0, 1, 1),  # 256: one set
 ]
 
 
