@@ -792,7 +792,7 @@ def traffic_summary(d: Path, batch: int, policy: str, commands: list) -> dict:
     fetch_b = per["FETCH_SIZE"][1] * 1024 * f_fetch
     write_b = per["WRITE_SIZE"][1] * 1024 * f_write
     return {
-        "kernel": f"conv_igemm_kernel / conv_igemm_sk_kernel / stem7_mfma_kernel (all instantiations), implicit-GEMM layers of "
+        "kernel": f"conv_igemm_kernel / conv_igemm_sk_kernel / conv_split_kernel / stem7_mfma_kernel (all instantiations), implicit-GEMM layers of "
                   f"ResNet-101 v1.5 fp32 "
                   f"batch {batch}",
         "conv_policy": policy, "batch": batch, "commands": commands,
@@ -1430,7 +1430,7 @@ def main() -> int:
         "roofline": {"bound": "mfma", "achieved": round(ig_tflops, 3), "peak": PEAK_FP32_MFMA / 1e12,
                      "unit": "TFLOP/s", "frac": round(ig_tflops * 1e12 / PEAK_FP32_MFMA, 4),
                      "traffic": measured_traffic(a.batch, a.policy),
-                     "kernel": f"conv_igemm_kernel / conv_igemm_sk_kernel / stem7_mfma_kernel (implicit-GEMM conv, {n_ig} layers, "
+                     "kernel": f"conv_igemm_kernel / conv_igemm_sk_kernel / conv_split_kernel / stem7_mfma_kernel (implicit-GEMM conv, {n_ig} layers, "
                                f"batch {a.batch})",
                      "launch_us": round(ig_live_ms / max(n_ig, 1) * 1e3, 2),
                      "achieved_node_events": round(ig_node_tflops, 3),
