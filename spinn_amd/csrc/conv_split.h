@@ -52,6 +52,7 @@ struct SplitPw2 {
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t off; // byte offset of the thread's first pixel at channel 0; kOOB past the last
     uint32_t hw4;
+    uint32_t lost = 0; // split2
     int oct;      // channel octet of the next fetch
     int co8;
     struct Stage {
@@ -74,9 +75,9 @@ struct SplitPw2 {
         for (int e = 0; e < 8; ++e) buf_load_cw<2>(rsrc, v, (uint32_t)e * hw4, st.r[e]);
         oct += 4 * kSplitGS;
     }
-    __device__ __forceinline__ void split(const Stage &st, int i, int q, u32x4 (&p)[3]) const {
+    __device__ __forceinline__ void split(const Stage &st, int i, int q, u32x4 (&p)[3]) {
         uint32_t h, m, l;
-        split2(st.r[2 * q][i], st.r[2 * q + 1][i], h, m, l);
+        split2(st.r[2 * q][i], st.r[2 * q + 1][i], h, m, l, lost);
         p[0][q] = h;
         p[1][q] = m;
         p[2][q] = l;
@@ -97,6 +98,7 @@ struct SplitGather {
     uint32_t off; // byte offset of (image, group channel 0, window origin)
     int ih0, iw0; // window origin; ih0 far outside the image past the last pixel
     uint32_t hw4;
+    uint32_t lost = 0; // split2
     int H, W, KH, KW, Cg, co8;
     int co[kSplitGS], kh[kSplitGS], kw[kSplitGS]; // next octet to fetch
     struct Stage {
@@ -152,14 +154,14 @@ struct SplitGather {
             }
         }
     }
-    __device__ __forceinline__ void split(const Stage &st, int i, int q, u32x4 (&p)[3]) const {
+    __device__ __forceinline__ void split(const Stage &st, int i, int q, u32x4 (&p)[3]) {
         float v0 = st.r[i][2 * q], v1 = st.r[i][2 * q + 1];
         if constexpr (TAIL) {
             v0 = 2 * q < st.live[i] ? v0 : 0.f;
             v1 = 2 * q + 1 < st.live[i] ? v1 : 0.f;
         }
         uint32_t h, m, l;
-        split2(v0, v1, h, m, l);
+        split2(v0, v1, h, m, l, lost);
         p[0][q] = h;
         p[1][q] = m;
         p[2][q] = l;
@@ -235,12 +237,70 @@ __device__ __forceinline__ void split_store(const ConvKArgs &a, int group, int m
     }
 }
 
+// A wave's accumulators again on the fp32 MFMA, from the packed fp32 weights, an octet of k
+// ahead of its loads' use. Where one wave of a tile has to, it takes about three times the
+// time (1x1 1024 -> 256@14x14 at batch 32: 29.5 -> 97 us; with a division per element and
+// no loads ahead 177); all waves at once 105 us.
+template <class T, bool RES>
+__device__ __forceinline__ void split_redo(const ConvSplitArgs &a, int group, int m0, int n0, int g0, int g1, bool terms,
+                                           f32x4 (&acc)[T::TM][T::TN], int lane) {
+    split_acc_start<T, RES>(a.t, group, m0, n0, lane, terms, acc);
+    const ConvGeom &cg = a.t.geom;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(cg.x, cg.x_bytes);
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.t.wpk + group * a.t.wpk_group_stride, (uint32_t)a.t.wpk_group_stride * 4u);
+    const int taps = cg.KH * cg.KW;
+    const uint32_t hw4 = (uint32_t)(cg.H * cg.W) * 4u;
+    const int k4 = lane >> 4;
+    uint32_t off[T::TN]; // byte offset of (image, group channel 0, window origin)
+    int ih0[T::TN], iw0[T::TN];
+#pragma unroll
+    for (int j = 0; j < T::TN; ++j) {
+        PixelOrigin px;
+        px.init(cg, n0 + T::col0(j % T::NQ, lane) + j / T::NQ, group);
+        ih0[j] = px.valid ? px.ih0 : INT32_MIN / 2;
+        iw0[j] = px.iw0;
+        off[j] = (px.base + (uint32_t)(px.ih0 * cg.W + px.iw0)) * 4u;
+    }
+    const int o0 = g0 * (4 * kSplitGS), o1 = min(g1 * (4 * kSplitGS), taps * a.co8);
+    int tap = o0 / a.co8, co = o0 - tap * a.co8;
+    int kh = tap / cg.KW, kw = tap - kh * cg.KW;
+    // octets come in order; those past the last read zeros
+    auto load = [&](int, float (&va)[2][T::TM], float (&vb)[2][T::TN]) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int c = co * 8 + 4 * s + k4;
+            const bool ok = (tap < taps) & (c < cg.Cg);
+            const uint32_t k = (uint32_t)(a.tap_order ? tap * cg.Cg + c : c * taps + tap);
+#pragma unroll
+            for (int i = 0; i < T::TM; ++i) {
+                const int m = m0 + i * 16 + (lane & 15);
+                va[s][i] = buf_f32(rw, ok & (m < a.t.M) ? (k * (uint32_t)a.t.ldw + (uint32_t)m) * 4u : kOOB);
+            }
+#pragma unroll
+            for (int j = 0; j < T::TN; ++j) {
+                const int ih = ih0[j] + kh, iw = iw0[j] + kw;
+                const bool in = ok & ((unsigned)ih < (unsigned)cg.H) & ((unsigned)iw < (unsigned)cg.W);
+                vb[s][j] = buf_f32(rx, in ? off[j] + (uint32_t)(kh * cg.W + kw) * 4u + (uint32_t)c * hw4 : kOOB);
+            }
+        }
+        if (++co == a.co8) {
+            co = 0;
+            ++tap;
+            if (++kw == cg.KW) {
+                kw = 0;
+                ++kh;
+            }
+        }
+    };
+    fp32_product<T::TM, T::TN>(o0, o1, acc, load);
+}
+
 // Groups [g0, g1) (of GS slices) of one output tile into acc; m0: the wave's first row,
-// n0 the tile's first column.
+// n0 the tile's first column. lost (LDS): the bits that each thread's activations lost.
 template <class T, class BL, bool RES>
 __device__ __forceinline__ void split_conv_segment(const ConvSplitArgs &a, int group, int m0, int n0, int g0, int g1,
                                                    bool terms, u32x4 (*lds)[kSplitRuns],
-                                                   f32x4 (&acc)[T::TM][T::TN], int tid, int lane) {
+                                                   uint32_t *lost, f32x4 (&acc)[T::TM][T::TN], int tid, int lane) {
     constexpr int GS = kSplitGS;
     SplitPlanes w = a.w;
     w.base = (const float *)((const char *)w.base + group * a.w_group_stride);
@@ -315,6 +375,7 @@ __device__ __forceinline__ void split_conv_segment(const ConvSplitArgs &a, int g
             al.fetch(g * GS + sl + 2, wa[w_]);
             SPINN_FENCE;
         }
+        lost[tid] = bl.lost; // of group g + 1 and all before it
         __syncthreads();
     };
 #undef SPINN_FENCE
@@ -329,28 +390,22 @@ __device__ __forceinline__ void split_conv_segment(const ConvSplitArgs &a, int g
     for (int i = 0; i < T::TM; ++i)
 #pragma unroll
         for (int j = 0; j < T::TN; ++j) acc[i][j] += low[i][j];
-    if (out_of_range<T::TM, T::TN>(acc)) {
-        split_acc_start<T, RES>(a.t, group, m0, n0, lane, terms, acc);
-        const ConvGeom &cg = a.t.geom;
-        const __amdgpu_buffer_rsrc_t rx = make_rsrc(cg.x, cg.x_bytes);
-        const float *wt = a.t.wpk + group * a.t.wpk_group_stride;
-        const int taps = cg.KH * cg.KW;
-        auto av = [&](int i, int k) {
-            const int tap = (k >> 3) / a.co8, c = k - tap * a.co8 * 8;
-            const int m = m0 + i * 16 + (lane & 15);
-            const bool ok = m < a.t.M && tap < taps && c < cg.Cg;
-            return ok ? wt[(int64_t)(a.tap_order ? tap * cg.Cg + c : c * taps + tap) * a.t.ldw + m] : 0.f;
-        };
-        auto bv = [&](int j, int k) {
-            PixelOrigin px;
-            px.init(cg, n0 + T::col0(j % T::NQ, lane) + j / T::NQ, group);
-            const int tap = (k >> 3) / a.co8, c = k - tap * a.co8 * 8;
-            const int kh = tap / cg.KW;
-            const int ih = px.ih0 + kh, iw = px.iw0 + tap - kh * cg.KW;
-            const bool ok = px.valid && tap < taps && c < cg.Cg && (unsigned)ih < (unsigned)cg.H && (unsigned)iw < (unsigned)cg.W;
-            return buf_f32(rx, ok ? (px.base + (uint32_t)c * (uint32_t)(cg.H * cg.W) + (uint32_t)(ih * cg.W + iw)) * 4u : kOOB);
-        };
-        fp32_product<T::TM, T::TN>(g0 * GS * kSplitBK, g1 * GS * kSplitBK, lane, acc, av, bv);
+}
+
+// Computes a finished segment again where bf16 parts could not carry it (split_core.h); lost:
+// the segment's notes. `after` follows where sums were replaced. The indexes are copies that
+// the compiler cannot tell from new ones: it would keep what this shares with the prologue
+// in registers over the K loop.
+template <class T, bool RES, class After>
+__device__ __forceinline__ void split_check(const ConvSplitArgs &a, int group, int m0, int n0, int g0, int g1, bool terms,
+                                            f32x4 (&acc)[T::TM][T::TN], const uint32_t *lost, int lane, const After &after) {
+    if (__builtin_expect(__any(sums_suspect<T::TM, T::TN>(acc)), 0)) {
+        asm volatile("" : "+v"(lane), "+s"(m0), "+s"(n0));
+        const uint32_t bits = lost[lane] | lost[64 + lane] | lost[128 + lane] | lost[192 + lane];
+        if (__any(sums_bad<T::TM, T::TN>(acc) | ((bits & 0xffffu) != 0u))) {
+            split_redo<T, RES>(a, group, m0, n0, g0, g1, terms, acc, lane);
+            after();
+        }
     }
 }
 
@@ -363,6 +418,7 @@ __device__ __forceinline__ void split_conv_segment(const ConvSplitArgs &a, int g
 template <class T, class BL, bool RES, int AC, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 2) void conv_split_kernel(ConvSplitArgs a) {
     __shared__ u32x4 lds[2][kSplitRuns];
+    __shared__ uint32_t lost[kThreads];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -375,39 +431,53 @@ __global__ __launch_bounds__(kThreads, 2) void conv_split_kernel(ConvSplitArgs a
     const int g0 = SPLIT ? z * a.chunk : 0;
     const int g1 = SPLIT ? min(a.groups_k, g0 + a.chunk) : a.groups_k;
     f32x4 acc[T::TM][T::TN];
-    split_conv_segment<T, BL, RES>(a, group, m0, n0, g0, g1, !SPLIT, lds, acc, tid, lane);
-    if constexpr (SPLIT) {
-        const int ntot = a.t.geom.ntot;
+    split_conv_segment<T, BL, RES>(a, group, m0, n0, g0, g1, !SPLIT, lds, lost, acc, tid, lane);
+    auto store = [&] {
+        if constexpr (SPLIT) {
+            const int ntot = a.t.geom.ntot;
 #pragma unroll
-        for (int j = 0; j < T::TN; ++j) {
-            const int jcol = n0 + T::col0(j % T::NQ, lane) + j / T::NQ;
-            if (jcol >= ntot) continue;
-            float *wsz = a.t.ws + (int64_t)z * a.t.OC * ntot + jcol;
+            for (int j = 0; j < T::TN; ++j) {
+                const int jcol = n0 + T::col0(j % T::NQ, lane) + j / T::NQ;
+                if (jcol >= ntot) continue;
+                float *wsz = a.t.ws + (int64_t)z * a.t.OC * ntot + jcol;
 #pragma unroll
-            for (int i = 0; i < T::TM; ++i)
+                for (int i = 0; i < T::TM; ++i)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int m = m0 + i * 16 + 4 * (lane >> 4) + r;
-                    if (m < a.t.M) wsz[(int64_t)m * ntot] = acc[i][j][r];
-                }
+                    for (int r = 0; r < 4; ++r) {
+                        const int m = m0 + i * 16 + 4 * (lane >> 4) + r;
+                        if (m < a.t.M) wsz[(int64_t)m * ntot] = acc[i][j][r];
+                    }
+            }
+        } else {
+            split_store<T, AC>(a.t, group, m0, n0, lane, acc);
         }
-    } else {
-        split_store<T, AC>(a.t, group, m0, n0, lane, acc);
-    }
+    };
+    // Stored first, so that the check runs while the stores drain, and once more where sums
+    // were replaced; not with a residual, which the output may be written over.
+    if constexpr (!RES) store();
+    split_check<T, RES>(a, group, m0, n0, g0, g1, !SPLIT, acc, lost, lane, [&] {
+        if constexpr (!RES) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            store();
+        }
+    });
+    if constexpr (RES) store();
 }
 
 // Data-parallel + stream-K launch (streamk.h) of a group-1 conv.
 template <class T, class BL, bool RES, int AC, int SCHEME>
 __global__ __launch_bounds__(kThreads, 2) void conv_split_sk_kernel(ConvSplitArgs a, SkSched s) {
     __shared__ u32x4 lds[2][kSplitRuns];
+    __shared__ uint32_t lost[kThreads];
     __shared__ int sk_last;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     typedef f32x4 Acc[T::TM][T::TN];
     auto segment = [&](int t, int k0, int k1, Acc &acc) {
-        split_conv_segment<T, BL, RES>(a, 0, (t % s.tiles_m) * T::BM + wave * T::WM, (t / s.tiles_m) * kSplitBN, k0,
-                                       k1, k0 == 0, lds, acc, tid, lane);
+        const int m0 = (t % s.tiles_m) * T::BM + wave * T::WM, n0 = (t / s.tiles_m) * kSplitBN;
+        split_conv_segment<T, BL, RES>(a, 0, m0, n0, k0, k1, k0 == 0, lds, lost, acc, tid, lane);
+        split_check<T, RES>(a, 0, m0, n0, k0, k1, k0 == 0, acc, lost, lane, [] {});
     };
     auto store = [&](int t, const Acc &acc) {
         split_store<T, AC>(a.t, 0, (t % s.tiles_m) * T::BM + wave * T::WM, (t / s.tiles_m) * kSplitBN, lane, acc);

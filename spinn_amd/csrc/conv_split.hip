@@ -8,8 +8,10 @@ namespace spinn {
 
 // W [group][OCg][Cg][KH][KW] -> split planes [group][octet][plane][rows_p][8], K in
 // (kh, kw, c) order, each tap's channels padded to octets; one thread per (octet, row).
+// An octet with a weight that loses bits, or of `limit` and more, gets a NaN, which sends its
+// row's tiles to the fp32 MFMA (split_core.h).
 __global__ void conv_pack_split_kernel(const float *__restrict__ w, u32x4 *__restrict__ out, int groups, int OCg,
-                                       int Cg, int KHW, int rows_p, int octs) {
+                                       int Cg, int KHW, int rows_p, int octs, float limit) {
     const int co8 = (Cg + 7) / 8;
     const int64_t total = (int64_t)groups * octs * rows_p;
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
@@ -21,10 +23,15 @@ __global__ void conv_pack_split_kernel(const float *__restrict__ w, u32x4 *__res
         const int tap = o / co8;
         const int c0 = (o - tap * co8) * 8;
         float v[8];
-        for (int i = 0; i < 8; ++i)
+        bool carried = true;
+        for (int i = 0; i < 8; ++i) {
             v[i] = (m < OCg && tap < KHW && c0 + i < Cg) ? w[((g * OCg + m) * Cg + c0 + i) * KHW + tap] : 0.f;
+            carried = carried && fabsf(v[i]) < limit;
+        }
         u32x4 p[3];
-        split8(v, p[0], p[1], p[2]);
+        uint32_t lost = 0;
+        split8(v, p[0], p[1], p[2], lost);
+        if (!carried || (lost & 0xffffu)) p[0][0] = 0x7fc0u;
         u32x4 *dst = out + (go * 3) * rows_p + m;
         for (int i = 0; i < 3; ++i) dst[(int64_t)i * rows_p] = p[i];
     }
@@ -151,7 +158,8 @@ int split_pack(const SpinnHipConvDesc *d, const float *w, float *packed, hipStre
     const int64_t total = (int64_t)d->group * split_octs(d) * split_rows(d);
     const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65535);
     hipLaunchKernelGGL(conv_pack_split_kernel, dim3(blocks), dim3(256), 0, st, w, (u32x4 *)packed, d->group,
-                       d->oc / d->group, d->c / d->group, d->kh * d->kw, split_rows(d), split_octs(d));
+                       d->oc / d->group, d->c / d->group, d->kh * d->kw, split_rows(d), split_octs(d),
+                       split_weight_limit(d->c / d->group * d->kh * d->kw));
     return check_launch();
 }
 

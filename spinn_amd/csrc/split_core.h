@@ -1,24 +1,34 @@
 // split_core.h - fp32 matrix products on the bf16 matrix cores (gfx950).
 //
-// An fp32 value is exactly the sum of three bf16 values: hi = bf16(v),
-// mid = bf16(v - hi), lo = bf16(v - hi - mid) (8 significant bits each, both
-// differences exact). A product a*b is then nine bf16 products, each exact in
-// fp32; the six largest are accumulated here, in fp32, by
-// v_mfma_f32_16x16x32_bf16. The three left out (mid*lo, lo*mid, lo*lo) are below
-// 2^-25 of |a*b|, under the rounding of the fp32 sums themselves. Six products at
-// 16x the fp32 MFMA rate leave 2.67x its throughput (157 -> 419 TFLOP/s peak).
+// An fp32 value is the sum of three bf16 values: hi = bf16(v), mid = bf16(v - hi), lo the
+// rest (8 significant bits each, both differences exact; from 2^-110 up the sum is exact,
+// below that low bits can fall under bf16's least number, 2^-133, and the sum is off by
+// less than that). A product a*b is then nine bf16 products, each exact in fp32; the six
+// largest are accumulated here, in fp32, by v_mfma_f32_16x16x32_bf16. Of the three left
+// out mid*lo and lo*mid are below 2^-25 of |a*b| each and lo*lo below 2^-34, so together
+// they can reach the half unit, 2^-24, by which a lone product is rounded (one-term sums:
+// largest error 1.65 x 2^-24, root mean square 0.435 x 2^-24 against 0.424 for fp32); sums
+// of 64 terms and more are closer to 64 bits than on the fp32 MFMA (split_mfma). Six
+// products at 16x the fp32 MFMA rate leave 2.67x its throughput (157 -> 419 TFLOP/s peak).
 //
-// Values that three bf16 parts cannot carry through a product turn every accumulator
-// they reach into NaN or infinity (infinities, NaN, magnitudes that round to infinity)
-// or leave it tiny (below 2^-110 the low parts fall under bf16's least number, 2^-133).
-// A wave that finds such an accumulator after its K loop computes all of its own again
-// on the fp32 MFMA (fp32_product), so these inputs give what fp32 arithmetic gives.
+// Operands that the parts cannot carry give what fp32 arithmetic gives: a wave that meets
+// them computes its accumulators again on the fp32 MFMA (fp32_product).
+//  * Infinities, NaN and magnitudes that round to infinity turn every accumulator they
+//    reach into an infinity or NaN.
+//  * Weights that lose bits (times activations of any size), or of split_weight_limit and
+//    more, are packed as NaN (conv_pack_split_kernel), which does the same.
+//  * Activations that lose bits are off by less than 2^-133 times a weight under the limit:
+//    over all of K by 2^-104 at most, 2^-24 of any accumulator of 2^-80 and more. Threads
+//    note whether they split one; where they did, accumulators below 2^-80, zeros among
+//    them, are computed again.
+//  * Nonzero accumulators below 2^-104 are computed again in any case: six products round
+//    at fp32's least number where fp32 rounds one.
 //
 // A operand (weights): split once when they are packed, laid out as the MFMA
 // reads them, [K/8][3 planes][rows][8 k]: each wave loads its rows' fragments
 // straight into registers, one 16-byte load per lane and plane.
 // B operand (activations): each thread loads 8 consecutive k of one column,
-// splits them (5.5 VALU operations per value) and stores three 16-byte runs to
+// splits them (6 VALU operations per value) and stores three 16-byte runs to
 // LDS, [octet of k][3 planes][columns (+2)][8 k]; the MFMA reads them back as
 // 16-byte fragments.
 #pragma once
@@ -52,24 +62,28 @@ struct SplitTiling {
     __device__ static __forceinline__ int col0(int q, int lane) { return (q * 16 + (lane & 15)) * CW; }
 };
 
-// Two values to their three bf16 parts, packed (first value in the low half).
-__device__ __forceinline__ void split2(float v0, float v1, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+// Two values to their three bf16 parts, packed (first value in the low half). The low 16 bits
+// of `lost` take what the parts leave out: for values they carry, lo is exactly the upper
+// half of what remains.
+__device__ __forceinline__ void split2(float v0, float v1, uint32_t &hi, uint32_t &mid, uint32_t &lo, uint32_t &lost) {
     const bf16x2 h = __builtin_convertvector((f32x2){v0, v1}, bf16x2);
     hi = __builtin_bit_cast(uint32_t, h);
     const float r0 = v0 - __builtin_bit_cast(float, hi << 16);
     const float r1 = v1 - __builtin_bit_cast(float, hi & 0xffff0000u);
     const bf16x2 m = __builtin_convertvector((f32x2){r0, r1}, bf16x2);
     mid = __builtin_bit_cast(uint32_t, m);
-    const float q0 = r0 - __builtin_bit_cast(float, mid << 16);
-    const float q1 = r1 - __builtin_bit_cast(float, mid & 0xffff0000u);
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){q0, q1}, bf16x2));
+    const uint32_t q0 = __builtin_bit_cast(uint32_t, r0 - __builtin_bit_cast(float, mid << 16));
+    const uint32_t q1 = __builtin_bit_cast(uint32_t, r1 - __builtin_bit_cast(float, mid & 0xffff0000u));
+    lo = __builtin_amdgcn_perm(q1, q0, 0x07060302u); // both upper halves
+    // by hand: as C the ORs are gathered into trees whose leaves stay in registers
+    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(q0), "v"(q1));
 }
 
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4 &hi, u32x4 &mid, u32x4 &lo) {
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4 &hi, u32x4 &mid, u32x4 &lo, uint32_t &lost) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t h, m, l;
-        split2(v[2 * i], v[2 * i + 1], h, m, l);
+        split2(v[2 * i], v[2 * i + 1], h, m, l, lost);
         hi[i] = h;
         mid[i] = m;
         lo[i] = l;
@@ -151,43 +165,78 @@ __device__ __forceinline__ void split_mfma(const bf16x8 (&a)[TM][3], const bf16x
         }
 }
 
-// True when any accumulator of the wave is infinite, NaN, or nonzero below 2^-80, which
-// sums of ordinary values do not cancel down to (their residue is 2^-24 of a term).
+// Magnitudes from which an accumulator outweighs the bits that activations lose (kSumLeast)
+// and below which six products round visibly more often than one (kSumUnder).
+constexpr float kSumLeast = 0x1p-80f, kSumUnder = 0x1p-104f;
+
+// Largest power of two that K weights below it keep under 2^29 in sum.
+inline float split_weight_limit(int K) {
+    int bits = 0;
+    while (((int64_t)1 << bits) < K) ++bits;
+    return __builtin_ldexpf(1.f, 29 - bits);
+}
+
+// Whether the lane holds an accumulator that is infinite, NaN, zero or below 2^-80 (zero is
+// also what outputs that do not exist hold).
 template <int TM, int TN>
-__device__ __forceinline__ bool out_of_range(const f32x4 (&acc)[TM][TN]) {
-    constexpr uint32_t kTiny = (127u - 80u) << 23;
-    float s = 0.f;         // v * 0 is 0 for finite v and NaN otherwise; a NaN survives the sums
-    uint32_t low = ~0u;    // least |v| - 1 as bits: zero wraps to the largest
+__device__ __forceinline__ bool sums_suspect(const f32x4 (&acc)[TM][TN]) {
+    float least = __builtin_inff(); // a NaN is passed over
+    float sum[2] = {0.f, 0.f};      // keeps an infinity or NaN, as one of the two or as inf - inf
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                least = fminf(least, fminf(fabsf(acc[i][j][r]), fabsf(acc[i][j][r + 1])));
+                sum[0] += acc[i][j][r];
+                sum[1] += acc[i][j][r + 1];
+            }
+    const float t = sum[0] + sum[1];
+    return !(fabsf(t) < __builtin_inff()) | (least < kSumLeast);
+}
+
+// Whether it holds an infinity, NaN or nonzero below 2^-104.
+template <int TM, int TN>
+__device__ __forceinline__ bool sums_bad(const f32x4 (&acc)[TM][TN]) {
+    bool bad = false;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                s += acc[i][j][r] * 0.f;
-                low = min(low, (__builtin_bit_cast(uint32_t, acc[i][j][r]) & 0x7fffffffu) - 1u);
+                const float v = fabsf(acc[i][j][r]);
+                bad = bad | !(v < __builtin_inff()) | ((v != 0.f) & (v < kSumUnder));
             }
-    return __any(s != s || low < kTiny);
+    return bad;
 }
 
-// Accumulators of one wave again in fp32: av(i, k) and bv(j, k) give the lane's
-// operand values for row block i and column block j.
-template <int TM, int TN, class AV, class BV>
-__device__ __forceinline__ void fp32_product(int k0, int k1, int lane, f32x4 (&acc)[TM][TN], const AV &av,
-                                             const BV &bv) {
+// Accumulators of one wave again in fp32, over octets of k: load(o, a, b) gives the lane's
+// operand values of octet o, a[s][i] for row block i and b[s][j] for column block j at
+// k = 8 * o + 4 * s + lane / 16. The next octet's loads are in flight under this one's
+// MFMAs.
+template <int TM, int TN, class Load>
+__device__ __forceinline__ void fp32_product(int o0, int o1, f32x4 (&acc)[TM][TN], Load &load) {
+    float a[2][TM], b[2][TN], an[2][TM], bn[2][TN];
+    if (o0 < o1) load(o0, a, b);
 #pragma unroll 1
-    for (int k = k0; k < k1; k += 4) {
-        const int kk = k + (lane >> 4);
-        float a[TM], b[TN];
+    for (int o = o0; o < o1; ++o) {
+        load(o + 1, an, bn);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = av(i, kk);
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) b[j] = bv(j, kk);
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][i], b[s][j], acc[i][j], 0, 0, 0);
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[s][i] = an[s][i];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[s][j] = bn[s][j];
+        }
     }
 }
 

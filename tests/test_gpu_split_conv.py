@@ -139,3 +139,69 @@ def test_split_conv_scales(hip, torch_gpu, tune, shape, sx, sw):
     rel = np.linalg.norm(y / scale - ref / scale) / np.linalg.norm(ref / scale)
     # fp32 sums of K terms in two-term steps on the fp32 path
     assert rel <= 2 * 2.0 ** -24 * (2 + math.sqrt(c * k * k / 2))
+
+
+@pytest.mark.parametrize("bm,split", [(64, 1), (128, 1), (64, 3), (128, 2)])
+@pytest.mark.parametrize("sx,sw", [(1e-36, 1e30), (1e30, 1e-36), (1e-37, 1e37), (1e37, 1e-37), (1e-40, 1e37),
+                                   (1e37, 1e-40), (1e-36, 1e14), (1e-42, 1e30), (1e-42, 1e4), (1.0, 1e-30)])
+@pytest.mark.parametrize("shape", [(2, 64, 7, 10, 65, 1, 1, 0, 1, 0), (1, 19, 10, 10, 80, 3, 1, 1, 1, 0),
+                                   (2, 256, 6, 6, 130, 1, 1, 0, 2, 0)], ids=["1x1", "3x3_tail", "grouped"])
+def test_split_conv_tiny_times_large(hip, torch_gpu, tune, shape, sx, sw, bm, split):
+    """Operands that three bf16 parts cannot hold, in ordinary sums: the other operand makes up
+    for them, or every part is zero."""
+    n, c, h, w, oc, k, s, p, g, act = shape
+    print(f"[split conv] {shape} x {sx} w {sw} bm {bm} split {split}", flush=True)
+    tune(1, bm, split)
+    x, wt, _, _ = _case(shape)
+    x, wt = (x * np.float32(sx)).astype(np.float32), (wt * np.float32(sw)).astype(np.float32)
+    d = conv_desc(hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch_gpu, d, x, wt)
+    ref = _exact(torch_gpu, shape, x, wt, np.zeros(oc, np.float32), None)
+    scale = ref.std()
+    rel = np.linalg.norm(y / scale - ref / scale) / np.linalg.norm(ref / scale)
+    # fp32 sums of K terms in two-term steps, and fp32's own least number in sums near it
+    kk = c // g * k * k
+    assert rel <= 2 * 2.0 ** -24 * (2 + math.sqrt(kk / 2)) + math.sqrt(kk) * 2.0 ** -149 / scale
+
+
+@pytest.mark.parametrize("bm,split", [(64, 1), (128, 1), (64, 2)])
+@pytest.mark.parametrize("k", [1, 3])
+def test_split_conv_tiny_operand_of_one_channel(hip, torch_gpu, tune, k, bm, split):
+    """One channel holds tiny inputs under large weights, or the reverse; the others are ordinary
+    but meet zeros, so the sums are the odd channel's alone and look like any others."""
+    n, c, hw, oc = 2, 96, 8, 128
+    tune(1, bm, split)
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((n, c, hw, hw)).astype(np.float32)
+    wt = rng.standard_normal((oc, c, k, k)).astype(np.float32)
+    x[:, ::2], wt[:, 1::2] = 0, 0           # every product is zero ...
+    x[:, 70] = rng.uniform(1, 2, x[:, 70].shape) * 2.0 ** -130
+    wt[:64, 70] *= np.float32(2.0 ** 100)   # ... but this channel's
+    wt[64:, 70] *= np.float32(2.0 ** 10)
+    x[0, 70] *= np.float32(2.0 ** 120)
+    wt[5, 70] *= np.float32(2.0 ** -225)
+    d = conv_desc(hip, n, c, hw, hw, oc, k, k, 1, 1, k // 2, k // 2, 1, 0, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch_gpu, d, x, wt)
+    shape = (n, c, hw, hw, oc, k, 1, k // 2, 1, 0)
+    ref = _exact(torch_gpu, shape, x, wt, np.zeros(oc, np.float32), None)
+    size = np.sqrt((ref ** 2).mean((2, 3), keepdims=True))  # per image and output channel
+    # nine terms at most; 2^-149 where a sum is that small
+    assert (np.abs(y - ref) <= 16 * 2.0 ** -24 * size + 9 * 2.0 ** -149).all()
+
+
+@pytest.mark.parametrize("bm", [64, 128])
+@pytest.mark.parametrize("hw", [8, 9])  # whole and ragged tiles; 2-pixel and 1-pixel loads
+@pytest.mark.parametrize("row", [16, 33, 50, 67])
+def test_split_conv_tiny_sums_of_one_row(hip, torch_gpu, tune, row, hw, bm):
+    """Tiny inputs that reach a single output channel, among channels of ordinary sums."""
+    n, c, oc = 1, 64, 128
+    tune(1, bm, 1)
+    rng = np.random.default_rng(row)
+    x = rng.standard_normal((n, c, hw, hw)).astype(np.float32)
+    wt = rng.standard_normal((oc, c, 1, 1)).astype(np.float32)
+    x[:, 9] = rng.uniform(1, 2, x[:, 9].shape) * 2.0 ** -126
+    wt[:, 9], wt[row], wt[row, 9] = 0, 0, 1.5
+    d = conv_desc(hip, n, c, hw, hw, oc, 1, 1, 1, 1, 0, 0, 1, 0, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch_gpu, d, x, wt)
+    ref = x[:, 9].astype(np.float64) * 1.5
+    assert (np.abs(y[:, row] - ref) <= 2.0 ** -149).all()
