@@ -113,10 +113,14 @@ SplitChoice split_choice(const SpinnHipConvDesc *d) {
     return c;
 }
 
+// Bytes of one group's planes.
+uint64_t split_plane_bytes(const SpinnHipConvDesc *d) { return (uint64_t)split_octs(d) * 3 * split_rows(d) * 16; }
+
 bool split_eligible(const SpinnHipConvDesc *d) {
-    // 16 channels: a slice's octets step at most two taps; the gathers' channel offsets
-    // stay inside the input
-    return d->c / d->group >= 16 && !stem_mfma_eligible(d);
+    // 16 channels: a fetch steps at most four taps (co8 >= 2), and the gathers' channel
+    // offsets stay inside the input. Planes are 1.5 times the weights: where they pass what
+    // one buffer descriptor spans, the fp32 kernels still run.
+    return d->c / d->group >= 16 && !stem_mfma_eligible(d) && split_plane_bytes(d) <= kMaxOperandBytes;
 }
 
 } // namespace
@@ -180,9 +184,7 @@ int split_conv(const SpinnHipConvDesc *d, const float *x, const float *wt, bool 
                float *y, void *ws, size_t ws_bytes, hipStream_t st) {
     const uint64_t x_bytes = (uint64_t)d->n * d->c * d->h * d->w * sizeof(float);
     const uint64_t y_bytes = (uint64_t)d->n * d->oc * d->oh * d->ow * sizeof(float);
-    const uint64_t w_bytes = (uint64_t)split_octs(d) * 3 * split_rows(d) * 16;
-    if (x_bytes > kMaxOperandBytes || y_bytes > kMaxOperandBytes || w_bytes > kMaxOperandBytes)
-        return SPINN_HIP_EUNSUPPORTED;
+    const uint64_t w_bytes = split_plane_bytes(d);
     const SplitChoice c = split_choice(d);
     ConvSplitArgs a{};
     a.t.M = d->oc / d->group;
@@ -192,6 +194,10 @@ int split_conv(const SpinnHipConvDesc *d, const float *x, const float *wt, bool 
     a.t.ldw = (a.t.M + 3) / 4 * 4;
     a.t.K = a.t.geom.Cg * d->kh * d->kw;
     a.t.wpk_group_stride = (int64_t)a.t.K * a.t.ldw;
+    // the limits of the fp32 kernels (conv_igemm.hip)
+    const uint64_t wt_bytes = (uint64_t)d->group * a.t.wpk_group_stride * sizeof(float);
+    if (x_bytes > kMaxOperandBytes || y_bytes > kMaxOperandBytes || wt_bytes > kMaxOperandBytes)
+        return SPINN_HIP_EUNSUPPORTED;
     a.tap_order = tap_order ? 1 : 0;
     a.t.y = y;
     a.t.bias = bias;

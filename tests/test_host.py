@@ -250,6 +250,19 @@ def test_conv_algo_selection(native):
     assert workspace(1, 512, 7, 7, 512, 3, 1, 1, 1) == 32 * 512 * 49 * 4
 
 
+def test_conv_planes_beyond_one_buffer_stay_off():
+    """Weights whose bf16 planes pass 2 GiB, though they themselves do not, keep the fp32
+    kernels alone: no planes are packed."""
+    L = native.lib()
+
+    def packed(c, oc, n=32):
+        d = native.ConvDesc(n, c, 14, 14, oc, 14, 14, 1, 1, 1, 1, 0, 0, 1, 0, native.ALGO_IMPLICIT_GEMM, 0)
+        return L.spinn_hip_conv_packed_size(C.byref(d))
+
+    assert packed(16384, 24576) == 16384 * 24576 * 4                       # planes of 2.25 GiB
+    assert packed(16384, 16384) == 16384 * 16384 * 4 + 16384 * 16384 * 6   # 1.5 GiB
+
+
 def _declared_functions():
     names = set()
     for h in (ROOT / "include").glob("*.h"):
