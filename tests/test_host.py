@@ -250,7 +250,7 @@ def test_conv_algo_selection(native):
     assert workspace(1, 512, 7, 7, 512, 3, 1, 1, 1) == 32 * 512 * 49 * 4
 
 
-def test_conv_planes_beyond_one_buffer_stay_off():
+def test_conv_planes_beyond_one_buffer_stay_off(native):
     """Weights whose bf16 planes pass 2 GiB, though they themselves do not, keep the fp32
     kernels alone: no planes are packed."""
     L = native.lib()
