@@ -132,7 +132,7 @@ void force_split_conv(int mode, int bm, int split) {
 }
 
 bool split_conv_selected(const SpinnHipConvDesc *d) {
-    if (!split_eligible(d) || tiles_forced()) return false;
+    if (!split_eligible(d) || tiles_forced() || wavek_forced_on()) return false;
     const int f = g_force_split.load();
     if (f >= 0) return f == 1;
     const int M = d->oc / d->group;

@@ -122,6 +122,7 @@ enum WkKind { kWkGemm, kWkConvGather, kWkConvPointwise }; // pointwise: 1x1 stri
 int wavek_tile(int M, int N, int K, int reps, WkKind kind);
 // true while spinn_hip_tune_force_tiles holds a tile shape or a K split
 bool tiles_forced();
+bool wavek_forced_on(); // SPINN_WAVEK=1: every shape on the wave-K kernel
 
 // 7x7 stride-2 stems (stem_mfma.hip): C <= 4, OC <= 64, output rows <= 128 pixels,
 // one workgroup per output row over an LDS-staged window; packed W^T as igemm_pack.

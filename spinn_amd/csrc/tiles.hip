@@ -32,6 +32,8 @@ static int env_wavek() {
     return v;
 }
 
+bool wavek_forced_on() { return env_wavek() == 1; }
+
 int wavek_tile(int M, int N, int K, int reps, WkKind kind) {
     if (g_force_bm) return (g_force_bm == g_force_bn && (g_force_bm == 32 || g_force_bm == 16)) ? g_force_bm : 0;
     const int e = env_wavek();

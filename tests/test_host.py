@@ -2,8 +2,11 @@
 (against the reference planner's offsets), the operator registry's error
 conventions and the exported C ABI. No GPU calls."""
 import ctypes as C
+import os
 import re
 import struct
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -261,6 +264,25 @@ def test_conv_planes_beyond_one_buffer_stay_off(native):
 
     assert packed(16384, 24576) == 16384 * 24576 * 4                       # planes of 2.25 GiB
     assert packed(16384, 16384) == 16384 * 16384 * 4 + 16384 * 16384 * 6   # 1.5 GiB
+
+
+def test_wavek_switch_covers_every_conv(native):
+    """SPINN_WAVEK=1 runs the wave-K kernel, which needs no workspace, for every implicit GEMM."""
+    code = """
+import ctypes as C
+from spinn_amd import native
+L = native.lib()
+for n, c, h, oc, k, s in ((32, 2048, 7, 512, 1, 1), (32, 1024, 14, 256, 1, 1), (32, 256, 28, 256, 3, 2)):
+    o = (h - 1) // s + 1
+    d = native.ConvDesc(n, c, h, h, oc, o, o, k, k, s, s, k // 2, k // 2, 1, 0, native.ALGO_IMPLICIT_GEMM, 0)
+    print(L.spinn_hip_conv_workspace_size(C.byref(d)))
+"""
+    sizes = {}
+    for v in ("", "1"):
+        r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=dict(os.environ, SPINN_WAVEK=v),
+                           capture_output=True, text=True, check=True)
+        sizes[v] = [int(x) for x in r.stdout.split()]
+    assert all(x > 0 for x in sizes[""]) and sizes["1"] == [0, 0, 0], sizes
 
 
 def _declared_functions():
