@@ -113,6 +113,12 @@ SplitChoice split_choice(const SpinnHipConvDesc *d) {
     return c;
 }
 
+// 1x1 convs that 2-pixel loads can serve (where the tensors are 8-byte aligned).
+bool split_pw2_shape(const SpinnHipConvDesc *d) {
+    return d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && d->ph == 0 && d->pw == 0 && d->oh == d->h &&
+           d->ow == d->w && (d->h * d->w) % 2 == 0 && d->c / d->group % 8 == 0;
+}
+
 // Bytes of one group's planes.
 uint64_t split_plane_bytes(const SpinnHipConvDesc *d) { return (uint64_t)split_octs(d) * 3 * split_rows(d) * 16; }
 
@@ -143,13 +149,33 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     // (64 -> 256@56x56 at batch 32: 42.0 -> 34.4) and loses with one (44.1 -> 47.3; K = 128,
     // 128 -> 512@28x28: 36.3 -> 38.8; K = 256, 256 -> 1024@14x14: 33.9 -> 32.4). Grids of
     // two thirds to one 64 x 64 tile per CU gain from K = 256 (384 -> 256@13x13 at batch 16:
-    // 13.4 -> 12.3; K = 128, 128@80x80 at batch 1: 6.06 and 6.09) and smaller ones lose
+    // 12.6 -> 12.4; K = 128, 128@80x80 at batch 1: 6.06 and 6.09) and smaller ones lose
     // (1024 -> 256@14x14 at batch 8: 15.8 on the wave-K kernel, 16.8 here), as do rows that
     // leave over a quarter of the tiles empty (80@80x80 at batch 1: 5.2 -> 5.9).
     const bool res = d->act == SPINN_ACT_ADD || d->act == SPINN_ACT_ADD_RELU;
     const int64_t cus = device_cu_count();
     if ((M + 63) / 64 * 64 * 3 > 4 * M || K < (res ? 256 : 64)) return false;
-    return tiles64 >= cus || (3 * tiles64 >= 2 * cus && K >= 256);
+    if (!(tiles64 >= cus || (3 * tiles64 >= 2 * cus && K >= 256))) return false;
+    // What the tiles do for padding counts against their rate: rows up to 64 or 128, and K up
+    // to whole groups of 64. Over 4000 shapes of 32-2048 channels, 7-112 pixels and batches of
+    // 1-32, against the kernels they had (fp32 tiles, split K, wave-K), at a real share of
+    //   under 0.7   0.93-1.19 of the time for 1x1 convs with 2-pixel loads, half of them
+    //               slower (96 -> 2016@16x16: K = 96 in two groups, 1.4), above it 0.79;
+    //   under 0.75  up to 1.47 for 1x1 convs with 1-pixel loads (64 -> 723@69x69 at batch 23:
+    //               167 -> 246), above it 0.84; 3x3 ones gain down to 0.65;
+    // and with 1-pixel loads one or two groups of K do not pay for their prologue (1.06).
+    const SplitChoice c = split_choice(d);
+    const int64_t rows = (M + c.bm - 1) / c.bm * c.bm, kpad = (int64_t)c.groups_k * kSplitGS * kSplitBK;
+    const int64_t real = (int64_t)M * K * 20, all = rows * kpad; // in twentieths
+    if (split_pw2_shape(d)) return real >= 14 * all;
+    if (real < (d->kh * d->kw > 1 ? 13 : 15) * all || c.groups_k < 3) return false;
+    if (c.bm == 128) return true;
+    // 64-row tiles, two to a CU, with 1-pixel loads: a little over one per CU, or two to three,
+    // leave most of the last round empty, where smaller fp32 tiles do not (112 -> 192 3x3
+    // stride 2, 273 tiles: 1.11; 176 -> 64, 601 tiles: 1.13); channel tails pay from one and
+    // a half per CU (614 -> 376, 216 tiles: 1.30).
+    if ((tiles64 > cus && 4 * tiles64 < 5 * cus) || (tiles64 > 2 * cus && tiles64 < 3 * cus)) return false;
+    return d->c / d->group % 8 == 0 || 2 * tiles64 >= 3 * cus;
 }
 
 int64_t split_packed_floats(const SpinnHipConvDesc *d) {
@@ -220,9 +246,7 @@ int split_conv(const SpinnHipConvDesc *d, const float *x, const float *wt, bool 
         a.t.ws = (float *)ws;
     }
     const SkSched *sk = c.sk ? &s : nullptr;
-    const bool pw2 = d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && d->ph == 0 && d->pw == 0 && d->oh == d->h &&
-                     d->ow == d->w && (d->h * d->w) % 2 == 0 && a.t.geom.Cg % 8 == 0 &&
-                     (((uintptr_t)x | (uintptr_t)y | (uintptr_t)res) & 7u) == 0;
+    const bool pw2 = split_pw2_shape(d) && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)res) & 7u) == 0;
     int rc;
     if (pw2) rc = launch_conv_split_pw2(a, c.bm, d->group, c.split, sk, c.sp.grid, st);
     else if (a.t.geom.Cg % 8 == 0) rc = launch_conv_split_gather(a, c.bm, d->group, c.split, sk, c.sp.grid, st);
