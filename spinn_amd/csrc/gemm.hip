@@ -31,10 +31,10 @@ struct GemmKArgs {
 
 // SETS: accumulator sets of the K loop. One chain over a K of some hundreds rounds more
 // than the wave-K kernel's eight; the grids that take 64 x 64 tiles in its place (under one
-// per CU, K of 128..576) use four, others one (2611 x 421 x 93, 287 tiles: 12.6 us with one
-// set, 14.0 with four) (the detector's attention at batch 16, two of whose
-// products these are: 4.3e-7 -> 2.9e-7 against 64 bits, 29.9 -> 30.7 us; 36.3 us with the
-// second product on the wave-K kernel).
+// per CU, K of 128..576: wavek_tile) use four, others one. The detector's attention at
+// batch 16, two of whose products these are: 4.3e-7 -> 2.9e-7 against 64 bits, 29.9 -> 30.7
+// us (36.3 us with the second product on the wave-K kernel). 2611 x 421 x 93, 287 tiles:
+// 12.6 us with one set, 14.0 with four.
 template <int BM, int BN, int BK, class ALoader, class BLoader, bool SPLIT, int SETS>
 __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmKArgs a) {
     using WT = WaveTiling<BM, BN>;

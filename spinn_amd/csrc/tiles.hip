@@ -83,13 +83,18 @@ int wavek_tile(int M, int N, int K, int reps, WkKind kind) {
     // per CU keeps the 64 x 64 tiles, unsplit (choose_tiles): ResNet-101 at batch 4,
     // 256 -> 1024@14x14 (208 tiles) 10.6 -> 8.4 us, 512 -> 1024@28x28 stride 2
     // 22.0 -> 15.8 us; YOLOv10n at batch 4, 192 -> 128@40x40 9.8 -> 7.0 us.
-    // So does a Gemm grid of half a 64 x 64 tile per CU (the detector's attention, 64 x 400 x
-    // 400: 32 of them, 224 tiles, 18.2 -> 12.5 us; 16 of them, 112 tiles, keep 9.0 against
-    // 10.6 us). A Gemm of at most one 16 x 16 tile per CU with K of 64..1024 takes those:
+    // A Gemm grid keeps them from 13/16 of a tile per CU where four fifths of the tiles are
+    // real (the detector's attention, 32 of 64 x 400 x 400: 224 tiles, 18.2 -> 12.5 us; 45
+    // such Gemms of 33-2048 rows and columns, K 128-576 and 1-64 batches 0.76 of the time,
+    // the worst 1.07). Fewer or emptier tiles, and the 32-row ones of M <= 32, lose as often as
+    // they gain (500 x 1500 x 300, 192 tiles: 9.6 -> 11.3; 32 x 400 x 400 of 32 up to 3.9
+    // times; 232 x 75 x 512 of 16, a Winograd layer: 22.1 -> 26.1).
+    // A Gemm of at most one 16 x 16 tile per CU with K of 64..1024 takes those:
     // 32 x 1000 x 512 6.3 -> 4.2 us, two of 64 x 400 x 400 5.1 -> 3.5 us; with more tiles
     // (eight of 64 x 400 x 400) the 32 x 32 ones keep 5.4 against 6.3 us.
     if (kind == kWkGemm && tiles16 <= cus && K >= 64 && K <= 1024) return 16;
-    if (kind == kWkGemm ? 2 * tiles64 >= cus : 2 * tiles64 > cus) return 0;
+    const bool real = 5 * (int64_t)M * N * reps >= 4 * tiles64 * 64 * 64;
+    if (kind == kWkGemm ? (M > 32 && 16 * tiles64 >= 13 * (int64_t)cus && real) : 2 * tiles64 > cus) return 0;
     return (K >= 128 && K <= 576) ? 32 : 0;
 }
 

@@ -24,6 +24,11 @@ GEMMS = [
     (500, 1000, 130, 1, 1, 1),   # 128 of them
     (960, 1088, 128, 0, 1, 1),   # 255: the most with four accumulator sets
     (1024, 1024, 128, 0, 1, 1),  # 256: one set
+    (832, 1024, 576, 0, 1, 1),   # 208: the fewest on 64 x 64 tiles
+    (832, 960, 576, 0, 0, 1),    # 195: 32 x 32 wave-K
+    (32, 8192, 128, 0, 1, 1),    # 32 rows: 32 x 32 wave-K
+    (32, 400, 400, 0, 1, 32),
+    (512, 1024, 512, 1, 0, 1),   # 128 tiles at K = 512: 32 x 32 wave-K, not split K
 ]
 
 

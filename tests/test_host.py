@@ -266,6 +266,14 @@ def test_conv_planes_beyond_one_buffer_stay_off(native):
     assert packed(16384, 16384) == 16384 * 16384 * 4 + 16384 * 16384 * 6   # 1.5 GiB
 
 
+def test_gemm_of_half_a_tile_per_cu_needs_no_workspace(native):
+    """Gemms of half a 64 x 64 tile per CU run on the wave-K kernel in one launch."""
+    L = native.lib()
+    for m, n, k in ((512, 1024, 512), (1024, 512, 576), (500, 1000, 520), (17, 8192, 512)):
+        d = native.GemmDesc(m, n, k, 0, 1, 0, 1.0, 0.0, 1, 0, 0, 0, 0)
+        assert L.spinn_hip_gemm_workspace_size(C.byref(d)) == 0, (m, n, k)
+
+
 def test_wavek_switch_covers_every_conv(native):
     """SPINN_WAVEK=1 runs the wave-K kernel, which needs no workspace, for every implicit GEMM."""
     code = """
