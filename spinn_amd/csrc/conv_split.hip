@@ -162,13 +162,15 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     //   under 0.7   0.93-1.19 of the time for 1x1 convs with 2-pixel loads, half of them
     //               slower (96 -> 2016@16x16: K = 96 in two groups, 1.4), above it 0.79;
     //   under 0.75  up to 1.47 for 1x1 convs with 1-pixel loads (64 -> 723@69x69 at batch 23:
-    //               167 -> 246), above it 0.84; 3x3 ones gain down to 0.65;
+    //               167 -> 246), above it 0.84; 3x3 ones gain down to 0.65, but past 64
+    //               rows not with K under four fifths of its groups (16 -> 304@83x83 at
+    //               batch 4: 33 -> 40);
     // and with 1-pixel loads one or two groups of K do not pay for their prologue (1.06).
     const SplitChoice c = split_choice(d);
     const int64_t rows = (M + c.bm - 1) / c.bm * c.bm, kpad = (int64_t)c.groups_k * kSplitGS * kSplitBK;
     const int64_t real = (int64_t)M * K * 20, all = rows * kpad; // in twentieths
     if (split_pw2_shape(d)) return real >= 14 * all;
-    if (real < (d->kh * d->kw > 1 ? 13 : 15) * all || c.groups_k < 3) return false;
+    if (real < (d->kh * d->kw > 1 ? 13 : 15) * all || c.groups_k < 3 || (M > 64 && 5 * K < 4 * kpad)) return false;
     if (c.bm == 128) return true;
     // 64-row tiles, two to a CU, with 1-pixel loads: a little over one per CU, or two to three,
     // leave most of the last round empty, where smaller fp32 tiles do not (112 -> 192 3x3
