@@ -52,6 +52,7 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "conv-layer fp32 GFLOP/s (% MFMA peak); ResNet-101 images/sec @ b1/b32, 1 GPU"
 PEAK_FP32_MFMA = 157.3e12  # MI355X dense fp32 matrix peak, FLOP/s
+PEAK_BF16_PARTS = PEAK_FP32_MFMA * 16 / 6  # fp32 products as six bf16 ones at 16 times the rate
 ALGO_NAMES = {1: "implicit_gemm", 2: "winograd", 3: "direct", 4: "winograd_f43"}
 
 
@@ -631,6 +632,13 @@ def executed_flops(r, algo: int) -> float:
 CONV_FIELDS = ("n", "c", "h", "w", "oc", "oh", "ow", "kh", "kw", "sh", "sw", "ph", "pw", "group", "act")
 
 
+def matrix_peak(N, row, algo: int) -> float:
+    """Peak FLOP/s of the matrix instructions that a conv layer runs on."""
+    import ctypes as C
+    d = N.ConvDesc(*(row[f] for f in CONV_FIELDS), algo, 0)
+    return PEAK_BF16_PARTS if N.lib().spinn_hip_conv_uses_bf16_parts(C.byref(d)) else PEAK_FP32_MFMA
+
+
 def conv_layers_live(N, rows, algo_for, reps: int = 10) -> list:
     """Live kernel time of every distinct conv layer shape in `rows`: launched through
     spinn_hip_conv with the algorithm `algo_for(row)` names, `reps` times back to back
@@ -638,8 +646,9 @@ def conv_layers_live(N, rows, algo_for, reps: int = 10) -> list:
     on, so the figure carries no host launch gap or event between the launches, unlike
     the per-node event pass.
     One entry per shape: the row, its count, algorithm, ms per launch (all of the
-    layer's kernels), direct and executed FLOPs and algorithmic bytes (input, weights,
-    bias, output, residual; fp32, each once)."""
+    layer's kernels), direct and executed FLOPs, the peak of the matrix instructions they
+    run on and algorithmic bytes (input, weights, bias, output, residual; fp32, each
+    once)."""
     import ctypes as C
     from spinn_amd.devbuf import DeviceBuffer, time_graph
     L = N.lib()
@@ -687,7 +696,8 @@ def conv_layers_live(N, rows, algo_for, reps: int = 10) -> list:
             byts = (nbytes(r["n"], r["c"], r["h"], r["w"]) + nbytes(r["oc"], r["c"] // r["group"], r["kh"], r["kw"])
                     + nbytes(r["oc"]) + nbytes(r["n"], r["oc"], r["oh"], r["ow"]) * (2 if has_res else 1))
             out.append(dict(row=r, count=len(rs), algo=algo, ms=ms, flops=r["flops"],
-                            exec_flops=executed_flops(r, algo), bytes=byts, split=ksplit))
+                            exec_flops=executed_flops(r, algo), peak=matrix_peak(N, r, algo), bytes=byts,
+                            split=ksplit))
             for buf in (pk, ws):
                 if buf:
                     buf.free()
@@ -714,32 +724,35 @@ def layers_markdown(live: list, batch: int, policy: str) -> str:
              "exec GFLOP = MFMA work actually issued (Winograd F(4x4,3x3): 36 GEMMs over 4x4 output tiles, "
              "transforms not counted). K split: split-K (partials reduced by a second launch) or stream-K "
              "(whole tiles plus the remaining tiles cut along K, finished in the same launch). "
-             "% peak against 157.3 TFLOP/s fp32 MFMA. Operands are random (uniform), never zero-filled. "
+             "Peak: 157.3 TFLOP/s fp32 MFMA, or 419.5 for layers whose fp32 products run as six bf16 ones. Operands are random (uniform), never zero-filled. "
              "MB = algorithmic bytes (input, weights, bias, output, residual, each once); bound = the longer of "
              "the direct FLOPs at MFMA peak and MB at 8 TB/s (executed FLOPs for Winograd), and % bound = that "
              "time over the measured one.", "",
-             "| layer (C,H,W -> OC, k/s, act) | x | algo | K split | GFLOP | exec GFLOP | MB | us / launch | "
+             "| layer (C,H,W -> OC, k/s, act) | x | algo | K split | peak TFLOP/s | GFLOP | exec GFLOP | MB | us / launch | "
              "TFLOP/s direct | % peak direct | % peak executed | bound | % bound |",
-             "|---|---|---|---|---|---|---|---|---|---|---|---|---|"]
-    tf = te = tt = 0.0
+             "|---|---|---|---|---|---|---|---|---|---|---|---|---|---|"]
+    tf = te = tt = td = tx = 0.0
     for e in live:
         r = e["row"]
         t = e["ms"] * 1e-3
         lines.append(f"| {r['c']},{r['h']},{r['w']} -> {r['oc']}, {r['kh']}x{r['kw']}/s{r['sh']}, {r['act']} | "
                      f"{e['count']} | {ALGO_NAMES.get(e['algo'], e['algo'])} | {e['split']} | "
+                     f"{e['peak'] / 1e12:.1f} | "
                      f"{e['flops'] / 1e9:.2f} | {e['exec_flops'] / 1e9:.2f} | {e['bytes'] / 1e6:.1f} | "
                      f"{e['ms'] * 1e3:.1f} | "
-                     f"{e['flops'] / t / 1e12:.1f} | {100 * e['flops'] / t / PEAK_FP32_MFMA:.1f} | "
-                     f"{100 * e['exec_flops'] / t / PEAK_FP32_MFMA:.1f} | "
-                     f"{'hbm' if e['bytes'] / 8e12 > e['exec_flops'] / PEAK_FP32_MFMA else 'mfma'} | "
-                     f"{100 * max(e['bytes'] / 8e12, e['exec_flops'] / PEAK_FP32_MFMA) / t:.1f} |")
+                     f"{e['flops'] / t / 1e12:.1f} | {100 * e['flops'] / t / e['peak']:.1f} | "
+                     f"{100 * e['exec_flops'] / t / e['peak']:.1f} | "
+                     f"{'hbm' if e['bytes'] / 8e12 > e['exec_flops'] / e['peak'] else 'mfma'} | "
+                     f"{100 * max(e['bytes'] / 8e12, e['exec_flops'] / e['peak']) / t:.1f} |")
         tf += e["flops"] * e["count"]
         te += e["exec_flops"] * e["count"]
         tt += e["ms"] * 1e-3 * e["count"]
+        td += e["flops"] / e["peak"] * e["count"]
+        tx += e["exec_flops"] / e["peak"] * e["count"]
     lines += ["", f"All {sum(e['count'] for e in live)} conv layers: {tt * 1e3:.3f} ms of kernel time, "
                   f"{tf / 1e9:.1f} GFLOP direct ({tf / tt / 1e12:.1f} TFLOP/s, "
-                  f"{100 * tf / tt / PEAK_FP32_MFMA:.1f} % of peak), {te / 1e9:.1f} GFLOP executed "
-                  f"({te / tt / 1e12:.1f} TFLOP/s, {100 * te / tt / PEAK_FP32_MFMA:.1f} % of peak)."]
+                  f"{100 * td / tt:.1f} % of the layers' peaks), {te / 1e9:.1f} GFLOP executed "
+                  f"({te / tt / 1e12:.1f} TFLOP/s, {100 * tx / tt:.1f} %)."]
     return "\n".join(lines) + "\n"
 
 
@@ -763,12 +776,17 @@ def igemm_algorithmic_bytes(batch: int, policy: str) -> float:
     return sum(alg) / len(alg)
 
 
+# the kernels that implicit-GEMM layers of ResNet-101 run on at batch 32: fp32 tiles and their
+# data-parallel + stream-K form, the same on the bf16 matrix cores, the 7x7 stem
+IGEMM_KERNELS = ("conv_igemm_kernel", "conv_igemm_sk_kernel", "conv_split_kernel", "conv_split_sk_kernel",
+                 "stem7_mfma_kernel")
+
+
 def traffic_summary(d: Path, batch: int, policy: str, commands: list) -> dict:
     """Reduce the four rocprofv3 --pmc counter CSVs under `d` (calib_{FETCH,WRITE}_SIZE
     from the calibration kernels, r101_{FETCH,WRITE}_SIZE from --profile-pass) to
-    calibrated HBM-side bytes per implicit-GEMM conv dispatch (conv_igemm_kernel, its
-    data-parallel + stream-K form conv_igemm_sk_kernel and the 7x7 stem's stem7_mfma_kernel;
-    split-K reductions not counted)."""
+    calibrated HBM-side bytes per implicit-GEMM conv dispatch (IGEMM_KERNELS; split-K
+    reductions not counted)."""
     import csv
 
     def rows(name):
@@ -787,12 +805,12 @@ def traffic_summary(d: Path, batch: int, policy: str, commands: list) -> dict:
     per = {}
     for counter in ("FETCH_SIZE", "WRITE_SIZE"):
         v = [x for n, x in rows(f"r101_{counter}")
-             if "conv_igemm_kernel" in n or "conv_igemm_sk_kernel" in n or "stem7_mfma_kernel" in n]
+             if any(k in n for k in IGEMM_KERNELS)]
         per[counter] = (len(v), sum(v) / len(v))
     fetch_b = per["FETCH_SIZE"][1] * 1024 * f_fetch
     write_b = per["WRITE_SIZE"][1] * 1024 * f_write
     return {
-        "kernel": f"conv_igemm_kernel / conv_igemm_sk_kernel / conv_split_kernel / stem7_mfma_kernel (all instantiations), implicit-GEMM layers of "
+        "kernel": f"{' / '.join(IGEMM_KERNELS)} (all instantiations), implicit-GEMM layers of "
                   f"ResNet-101 v1.5 fp32 "
                   f"batch {batch}",
         "conv_policy": policy, "batch": batch, "commands": commands,
@@ -885,9 +903,9 @@ def roofline_trace_summary(trace: Path, pass_json: Path) -> str:
             in_pack = True
             continue
         in_pack = False
-        if cur is None or not name.startswith(("conv_igemm", "conv_splitk_reduce", "stem7_mfma")):
-            continue
         base = name.split("<")[0]
+        if cur is None or base not in IGEMM_KERNELS + ("conv_splitk_reduce_kernel",):
+            continue
         if cur["main"] is None:
             cur["main"] = base
         if base == cur["main"]:
@@ -1283,10 +1301,11 @@ def main() -> int:
         fl = sum(e["flops"] * e["count"] for e in live)
         n = sum(e["count"] for e in live)
         tf = fl / (ms * 1e-3) / 1e12
+        peak = fl / sum(e["flops"] / e["peak"] * e["count"] for e in live)
         lab = lambda r: f"{r['c']},{r['h']},{r['w']} -> {r['oc']}, {r['kh']}x{r['kw']}/s{r['sh']}, {r['act']}"  # noqa: E731
         print(json.dumps({"roofline_pass": True, "batch": a.batch, "layers": n, "launch_us": round(ms / n * 1e3, 2),
                           "gflop_per_launch": fl / n / 1e9, "achieved": round(tf, 3),
-                          "frac": round(tf * 1e12 / PEAK_FP32_MFMA, 4),
+                          "frac": round(tf * 1e12 / peak, 4),
                           "shapes": [{"layer": lab(e["row"]), "count": e["count"], "us": round(e["ms"] * 1e3, 3),
                                       "split": e["split"]} for e in live]}))
         return 0
@@ -1350,7 +1369,7 @@ def main() -> int:
 
     rows = conv_table(gB)
     layers = []
-    tot_f = tot_t = ig_f = ig_t = 0.0
+    tot_f = tot_t = tot_p = ig_f = ig_t = 0.0
     n_ig = 0
     for r in rows:
         ms = float(node_ms[r["node"]])
@@ -1358,7 +1377,8 @@ def main() -> int:
         gf = r["flops"] / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
         layers.append(dict(node=r["node"], shape=f"{r['c']}x{r['h']}x{r['w']}->{r['oc']}x{r['oh']}x{r['ow']}",
                            k=f"{r['kh']}x{r['kw']}/s{r['sh']}", act=r["act"], algo=ALGO_NAMES.get(algo, str(algo)),
-                           gflop=r["flops"] / 1e9, ms=ms, gflops=gf, frac_peak=gf * 1e9 / PEAK_FP32_MFMA))
+                           gflop=r["flops"] / 1e9, ms=ms, gflops=gf, frac_peak=gf * 1e9 / matrix_peak(N, r, algo)))
+        tot_p += r["flops"] / matrix_peak(N, r, algo)
         tot_f += r["flops"]
         tot_t += ms
         if algo == N.ALGO_IMPLICIT_GEMM:
@@ -1373,12 +1393,17 @@ def main() -> int:
     ig_live_ms = sum(e["ms"] * e["count"] for e in ig_live)
     ig_live_f = sum(e["flops"] * e["count"] for e in ig_live)
     ig_tflops = ig_live_f / (ig_live_ms * 1e-3) / 1e12 if ig_live_ms > 0 else ig_node_tflops
+    # the peak of the matrix instructions each layer runs on (fp32 MFMA, or six bf16 products)
+    ig_peak_s = sum(e["flops"] / e["peak"] * e["count"] for e in ig_live)
+    ig_peak = ig_live_f / ig_peak_s if ig_peak_s > 0 else PEAK_FP32_MFMA
     # each layer's own roofline: MFMA time or HBM time (algorithmic bytes at 8 TB/s), whichever is longer
-    ig_bound_ms = sum(max(e["flops"] / PEAK_FP32_MFMA, e["bytes"] / 8e12) * 1e3 * e["count"] for e in ig_live)
-    ig_hbm_layers = sum(e["count"] for e in ig_live if e["bytes"] / 8e12 > e["flops"] / PEAK_FP32_MFMA)
+    ig_bound_ms = sum(max(e["flops"] / e["peak"], e["bytes"] / 8e12) * 1e3 * e["count"] for e in ig_live)
+    ig_hbm_layers = sum(e["count"] for e in ig_live if e["bytes"] / 8e12 > e["flops"] / e["peak"])
     live_ms = sum(e["ms"] * e["count"] for e in live)
     live_f = sum(e["flops"] * e["count"] for e in live)
     live_ef = sum(e["exec_flops"] * e["count"] for e in live)
+    live_p = sum(e["flops"] / e["peak"] * e["count"] for e in live)
+    live_ep = sum(e["exec_flops"] / e["peak"] * e["count"] for e in live)
     print(f"[bench] implicit-GEMM kernels: {ig_live_ms:.3f} ms per pass back to back "
           f"({ig_tflops:.1f} TFLOP/s), {ig_t:.3f} ms in the per-node event pass ({ig_node_tflops:.1f}); "
           f"all conv kernels {live_ms:.3f} ms", file=sys.stderr, flush=True)
@@ -1413,24 +1438,26 @@ def main() -> int:
         "ms_per_step_b1": round(ms_1, 4),
         "images_per_s_with_host_copies": round(a.batch / (ms_B_h2d * 1e-3), 2),
         "conv_tflops_aggregate": round(conv_tflops, 3),
-        "conv_frac_mfma_peak": round(conv_tflops * 1e12 / PEAK_FP32_MFMA, 4),
+        "conv_frac_mfma_peak": round(tot_p / (tot_t * 1e-3), 4),
         "conv_share_of_node_time": round(tot_t / all_ms, 4) if all_ms > 0 else None,
         "conv_kernels": {
             "ms_per_pass": round(live_ms, 4),
             "gflop_direct": round(live_f / 1e9, 2), "gflop_executed": round(live_ef / 1e9, 2),
             "tflops_direct_equiv": round(live_f / (live_ms * 1e-3) / 1e12, 2),
-            "frac_mfma_peak_direct_equiv": round(live_f / (live_ms * 1e-3) / PEAK_FP32_MFMA, 4),
+            "frac_mfma_peak_direct_equiv": round(live_p / (live_ms * 1e-3), 4),
             "tflops_executed": round(live_ef / (live_ms * 1e-3) / 1e12, 2),
-            "frac_mfma_peak_executed": round(live_ef / (live_ms * 1e-3) / PEAK_FP32_MFMA, 4),
+            "frac_mfma_peak_executed": round(live_ep / (live_ms * 1e-3), 4),
             "winograd_layers": sum(e["count"] for e in live if e["algo"] in (N.ALGO_WINOGRAD, N.ALGO_WINOGRAD_F43)),
             "method": "every conv layer's kernels launched 10x back to back in a HIP graph replayed between HIP "
                       "events; direct = "
                       "2*N*OC*OH*OW*C*KH*KW (Winograd credited at the direct count), executed = the MFMA work "
-                      "issued (Winograd: (m+2)^2 tile GEMMs, transforms not counted)"},
-        "roofline": {"bound": "mfma", "achieved": round(ig_tflops, 3), "peak": PEAK_FP32_MFMA / 1e12,
-                     "unit": "TFLOP/s", "frac": round(ig_tflops * 1e12 / PEAK_FP32_MFMA, 4),
+                      "issued (Winograd: (m+2)^2 tile GEMMs, transforms not counted); frac_mfma_peak: of the peak "
+                      "of the matrix instructions each layer runs on, 157.3 TFLOP/s fp32 MFMA or 419.5 as six "
+                      "bf16 products"},
+        "roofline": {"bound": "mfma", "achieved": round(ig_tflops, 3), "peak": round(ig_peak / 1e12, 3),
+                     "unit": "TFLOP/s", "frac": round(ig_tflops * 1e12 / ig_peak, 4),
                      "traffic": measured_traffic(a.batch, a.policy),
-                     "kernel": f"conv_igemm_kernel / conv_igemm_sk_kernel / conv_split_kernel / stem7_mfma_kernel (implicit-GEMM conv, {n_ig} layers, "
+                     "kernel": f"{' / '.join(IGEMM_KERNELS)} (implicit-GEMM conv, {n_ig} layers, "
                                f"batch {a.batch})",
                      "launch_us": round(ig_live_ms / max(n_ig, 1) * 1e3, 2),
                      "achieved_node_events": round(ig_node_tflops, 3),
@@ -1438,7 +1465,9 @@ def main() -> int:
                      "hbm_bound_layers": ig_hbm_layers,
                      "method": "direct-conv FLOPs of the implicit-GEMM layers / their kernel time, each "
                                "layer's kernel launched 10x back to back in a HIP graph replayed between HIP events, "
-                               "operands random (achieved_node_events: per-node events inside the model pass; "
+                               "operands random; peak: FLOPs over the time they take at the peak of the matrix "
+                               "instructions each layer runs on (157.3 TFLOP/s fp32 MFMA, 419.5 as six bf16 products) "
+                               "(achieved_node_events: per-node events inside the model pass; "
                                "frac_of_layer_rooflines: sum over the layers of max(FLOPs / MFMA peak, algorithmic "
                                "bytes / 8 TB/s) / their summed kernel time; hbm_bound_layers: layers whose bytes "
                                "take longer than their FLOPs at peak)"},

@@ -88,6 +88,9 @@ int spinn_hip_conv_noalloc(const SpinnHipConvDesc *d, const float *x, const floa
 
 /* Algorithm AUTO would run for this shape (never returns AUTO). */
 int spinn_hip_conv_select_algo(const SpinnHipConvDesc *d);
+/* 1 where spinn_hip_conv computes this descriptor's products on the bf16 matrix cores (each
+ * fp32 operand as three bf16 parts), else 0. No counterpart in the reference. */
+int spinn_hip_conv_uses_bf16_parts(const SpinnHipConvDesc *d);
 /* Device scratch bytes spinn_hip_conv needs for this descriptor (0 = none). */
 size_t spinn_hip_conv_workspace_size(const SpinnHipConvDesc *d);
 /* Bytes of pre-laid-out weights the selected algorithm needs (0 = reads w directly).

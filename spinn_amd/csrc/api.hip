@@ -114,6 +114,10 @@ int spinn_hip_conv_select_algo(const SpinnHipConvDesc *d) {
     return select_algo(d);
 }
 
+int spinn_hip_conv_uses_bf16_parts(const SpinnHipConvDesc *d) {
+    return conv_desc_ok(d) && select_algo(d) == SPINN_CONV_ALGO_IMPLICIT_GEMM && split_conv_selected(d) ? 1 : 0;
+}
+
 size_t spinn_hip_conv_workspace_size(const SpinnHipConvDesc *d) {
     if (!conv_desc_ok(d)) return 0;
     switch (select_algo(d)) {

@@ -133,6 +133,7 @@ _SIGS = {
     "spinn_hip_conv_noalloc": (C.c_int, [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                          C.c_void_p, C.c_void_p, C.c_void_p]),
     "spinn_hip_conv_select_algo": (C.c_int, [C.POINTER(ConvDesc)]),
+    "spinn_hip_conv_uses_bf16_parts": (C.c_int, [C.POINTER(ConvDesc)]),
     "spinn_hip_conv_workspace_size": (C.c_size_t, [C.POINTER(ConvDesc)]),
     "spinn_hip_conv_packed_size": (C.c_size_t, [C.POINTER(ConvDesc)]),
     "spinn_hip_conv_pack_weights": (C.c_int, [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p]),

@@ -266,6 +266,33 @@ def test_conv_planes_beyond_one_buffer_stay_off(native):
     assert packed(16384, 16384) == 16384 * 16384 * 4 + 16384 * 16384 * 6   # 1.5 GiB
 
 
+def test_conv_uses_bf16_parts(native):
+    """The convs that run on the bf16 matrix cores, at the edges of the rule."""
+    L = native.lib()
+
+    def parts(n, c, h, oc, k=1, s=1, g=1, act=0, algo=native.ALGO_AUTO):
+        o = (h + 2 * (k // 2) - k) // s + 1
+        d = native.ConvDesc(n, c, h, h, oc, o, o, k, k, s, s, k // 2, k // 2, g, act, algo, 0)
+        return L.spinn_hip_conv_uses_bf16_parts(C.byref(d))
+
+    assert parts(32, 1024, 14, 256) and parts(32, 256, 28, 256, 3, 2) and parts(32, 256, 14, 1024, act=5)
+    assert not parts(32, 128, 28, 512, act=5)      # a residual with K below 256
+    assert not parts(1, 1024, 14, 256)             # few tiles
+    assert not parts(32, 256, 28, 256, 3)          # Winograd
+    assert parts(32, 256, 28, 256, 3, algo=native.ALGO_IMPLICIT_GEMM)
+    assert not parts(32, 3, 224, 64, 7, 2)         # stem
+    assert parts(16, 64, 56, 256) and not parts(16, 64, 57, 256)      # one group of K: 2-pixel loads only
+    assert parts(16, 96, 40, 256) and not parts(16, 72, 40, 256)      # K = 96 and 72 of 128
+    assert parts(16, 192, 41, 256) and not parts(16, 136, 41, 256)    # K = 192 and 136 of 192, 1-pixel loads
+    # 64-row tiles with 1-pixel loads: 211 and 500 of them, not 263 or 605
+    assert parts(16, 176, 57, 64, 3, 2) and parts(38, 176, 57, 64, 3, 2)
+    assert not parts(20, 176, 57, 64, 3, 2) and not parts(46, 176, 57, 64, 3, 2)
+    assert not parts(16, 614, 29, 64) and parts(30, 614, 29, 64)      # a channel tail: 211, 395
+    assert not parts(4, 16, 83, 304, 3)            # K = 144 of 192
+    d = native.ConvDesc(1, 6, 8, 8, 4, 8, 8, 3, 3, 1, 1, 1, 1, 4, 0, 0, 0)
+    assert L.spinn_hip_conv_uses_bf16_parts(C.byref(d)) == 0          # refused
+
+
 def test_gemm_of_half_a_tile_per_cu_needs_no_workspace(native):
     """Gemms of half a 64 x 64 tile per CU run on the wave-K kernel in one launch."""
     L = native.lib()
@@ -381,16 +408,29 @@ def test_bench_roofline_trace_summary(tmp_path):
         k("void spinn::conv_igemm_sk_kernel<64, 64, 16, spinn::Pointwise1x1Loader<64, 16>, 1, 1>(spinn::ConvKArgs, "
           "spinn::SkSched)", 30.0)
     k("void spinn::xcc_id_kernel(unsigned int*)", 4.0)  # ignored
+    k("void spinn::conv_pack_wt_kernel(float const*, float*)", 2.0)
+    k("void spinn::conv_pack_split_kernel(float const*, unsigned int __vector(4)*, int)", 2.0)
+    for _ in range(4):  # shape 3: bf16 parts, split-K, 20 + 5 us per call
+        k("void spinn::conv_split_kernel<spinn::SplitTiling<128, 1>, spinn::SplitGather<false>, false, 0, true>("
+          "spinn::ConvSplitArgs)", 20.0)
+        k("void spinn::conv_splitk_reduce_kernel(float const*, int)", 5.0)
+    k("void spinn::conv_pack_split_kernel(float const*, unsigned int __vector(4)*, int)", 2.0)
+    for _ in range(4):  # shape 4: bf16 parts, stream-K
+        k("void spinn::conv_split_sk_kernel<spinn::SplitTiling<128, 2>, spinn::SplitPw2, true, 1, 1>("
+          "spinn::ConvSplitArgs, spinn::SkSched)", 40.0)
     lines = ["Kernel_Name,Start_Timestamp,End_Timestamp"] + [f'"{n}",{a},{b}' for n, a, b in rows]
     (tmp_path / "trace.csv").write_text("\n".join(lines) + "\n")
     (tmp_path / "pass.json").write_text(json.dumps({
         "launch_us": 26.0, "gflop_per_launch": 2.6, "achieved": 100.0,
-        "shapes": [{"layer": "a", "count": 1, "us": 12.0}, {"layer": "b", "count": 3, "us": 30.0}]}) + "\n")
+        "shapes": [{"layer": "a", "count": 1, "us": 12.0}, {"layer": "b", "count": 3, "us": 30.0},
+                   {"layer": "c", "count": 1, "us": 25.0}, {"layer": "d", "count": 1, "us": 40.0}]}) + "\n")
     md = bench.roofline_trace_summary(tmp_path / "trace.csv", tmp_path / "pass.json")
     assert "| a | 1 | conv_igemm_kernel | 4 | 12.00 | 12.00 | +0.0 % |" in md
     assert "| b | 3 | conv_igemm_sk_kernel | 4 | 30.00 | 30.00 | +0.0 % |" in md
-    # (12 * 1 + 30 * 3) / 4 = 25.5 us; 2.6 GFLOP / 25.5 us = 102.0 TFLOP/s
-    assert "rocprof 25.50 us, bench.py 25.50 us" in md and "rocprof 102.0 TFLOP/s" in md
+    assert "| c | 1 | conv_split_kernel | 4 | 25.00 | 25.00 | +0.0 % |" in md
+    assert "| d | 1 | conv_split_sk_kernel | 4 | 40.00 | 40.00 | +0.0 % |" in md
+    # (12 * 1 + 30 * 3 + 25 + 40) / 6 = 27.83 us; 2.6 GFLOP / 27.83 us = 93.4 TFLOP/s
+    assert "rocprof 27.83 us, bench.py 27.83 us" in md and "rocprof 93.4 TFLOP/s" in md
 
 
 def _hdr_fields(data):
