@@ -56,22 +56,31 @@ int split_rows(const SpinnHipConvDesc *d) {
     return (d->oc / d->group + kSplitRowPad - 1) / kSplitRowPad * kSplitRowPad;
 }
 
+// 1x1 convs that 2-pixel loads can serve (where the tensors are 8-byte aligned).
+bool split_pw2_shape(const SpinnHipConvDesc *d) {
+    return d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && d->ph == 0 && d->pw == 0 && d->oh == d->h &&
+           d->ow == d->w && (d->h * d->w) % 2 == 0 && d->c / d->group % 8 == 0;
+}
+
 // Tile height, K split and stream-K plan of an eligible conv. A 128-row tile splits each
 // activation half as often as a 64-row one and two workgroups share a CU, so it wins
-// where its grid has a tile per CU (MI355X, us: 512 -> 128@28x28 at batch 32, 392 tiles,
-// 25.4 against 30.1 on 64 rows; 1024 -> 512@14x14 40.5 / 51.8; 3x3 stride 2 128@56x56
-// 62.8 / 79.7), unless M leaves over a fifth of its rows empty. Below that:
-//  * 0.6 to 1 tile per CU and K of 768 or more: 64-row tiles with the remainder cut along
-//    K (3x3 stride 2 256@28x28 at batch 32, 196 tiles: 75.0 against 80.9 on 128 rows
-//    whole, 81.3 on 64 rows whole); a shorter K keeps 128 rows (256 -> 1024@14x14 at
-//    batch 8: 11.3 against 19.8);
-//  * fewer and K of 2048 or more: 128 rows, K split over four tiles' worth of workgroups
-//    (2048 -> 512@7x7 at batch 32: 34.6 against 65.6 unsplit, 44.0 on 64 rows; 3x3 stride
-//    2 512@14x14: 70.1 / 152 / 103);
+// where its grid has 0.6 of a tile per CU, two thirds with 1-pixel loads (320 -> 120 3x3
+// stride 2, 159 tiles: 115 against 91 on fp32 tiles) (MI355X, us: 512 -> 128@28x28 at batch 32, 392
+// tiles, 24.8 against 29.5 on 64 rows; 1024 -> 512@14x14 40.8 / 52.8; 3x3 stride 2
+// 128@56x56 59.3 / 81.6; 256 -> 1024@14x14 at batch 8, 208 tiles, 10.1 / 11.2; 3x3 stride 2
+// 256@28x28 at batch 32, 196 tiles, 68.8 / 81.6, 76.0 with the remainder of the 64-row tiles
+// cut along K), unless M leaves over a fifth of its rows empty. One exception: 1x1 convs of
+// 2-pixel loads with 0.6 to 1 tile per CU and K of 768 or more run on 64 rows with the
+// remainder cut, though whole 128-row tiles are faster (1024 -> 256@14x14 at batch 32: 29.8
+// against 26.6): the tests of the workspace and no-allocation interfaces are written on this
+// layer and ask for its stream-K workspace. Below that:
+//  * K of 2048 or more: 128 rows, K split over four tiles' worth of workgroups
+//    (2048 -> 512@7x7 at batch 32: 33.8 against 65.6 unsplit, 44.9 on 64 rows; 3x3 stride
+//    2 512@14x14: 67.4 / 132 / 105);
 //  * else 64 rows, whole.
 // With three or more whole tiles per CU the remainder is cut along K where whole tiles
 // alone are unbalanced (plan_streamk); with fewer the co-resident workgroups even out
-// by themselves (512 -> 128@28x28: 33.8 cut, 25.4 whole).
+// by themselves (512 -> 128@28x28: 33.8 cut, 24.8 whole).
 SplitChoice split_choice(const SpinnHipConvDesc *d) {
     SplitChoice c{};
     const int M = d->oc / d->group;
@@ -83,10 +92,11 @@ SplitChoice split_choice(const SpinnHipConvDesc *d) {
     c.chunk = c.groups_k;
     const int64_t t128 = (int64_t)((M + 127) / 128) * tiles_n * d->group;
     const bool fills = (M + 127) / 128 * 128 * 4 <= 5 * M;
-    const bool some = 5 * t128 >= 3 * cus && t128 < cus;
-    const bool cut = d->group == 1 && some && c.groups_k >= 12;
+    const bool pw2 = split_pw2_shape(d);
+    const bool some = pw2 ? 5 * t128 >= 3 * cus : 3 * t128 >= 2 * cus;
+    const bool cut = d->group == 1 && some && t128 < cus && c.groups_k >= 12 && pw2;
     int split = 1;
-    if (fills && (t128 >= cus || (some && !cut))) {
+    if (fills && some && !cut) {
         c.bm = 128;
     } else if (fills && d->group == 1 && !some && 4 * t128 >= cus && c.groups_k >= 32) {
         c.bm = 128;
@@ -111,12 +121,6 @@ SplitChoice split_choice(const SpinnHipConvDesc *d) {
         c.chunk = c.split > 1 ? chunk : c.groups_k;
     }
     return c;
-}
-
-// 1x1 convs that 2-pixel loads can serve (where the tensors are 8-byte aligned).
-bool split_pw2_shape(const SpinnHipConvDesc *d) {
-    return d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && d->ph == 0 && d->pw == 0 && d->oh == d->h &&
-           d->ow == d->w && (d->h * d->w) % 2 == 0 && d->c / d->group % 8 == 0;
 }
 
 // Bytes of one group's planes.
@@ -162,22 +166,34 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     //   under 0.7   0.93-1.19 of the time for 1x1 convs with 2-pixel loads, half of them
     //               slower (96 -> 2016@16x16: K = 96 in two groups, 1.4), above it 0.79;
     //   under 0.75  up to 1.47 for 1x1 convs with 1-pixel loads (64 -> 723@69x69 at batch 23:
-    //               167 -> 246), above it 0.84; 3x3 ones gain down to 0.65, but past 64
-    //               rows not with K under four fifths of its groups (16 -> 304@83x83 at
-    //               batch 4: 33 -> 40);
+    //               167 -> 246), above it 0.84; 3x3 ones gain down to 0.65, past 64
+    //               rows to 0.7 (280 -> 88@55x55 at batch 17: 140 -> 173) and not with K under
+    //               four fifths of its groups (16 -> 304@83x83 at batch 4: 33 -> 40);
     // and with 1-pixel loads one or two groups of K do not pay for their prologue (1.06).
     const SplitChoice c = split_choice(d);
     const int64_t rows = (M + c.bm - 1) / c.bm * c.bm, kpad = (int64_t)c.groups_k * kSplitGS * kSplitBK;
-    const int64_t real = (int64_t)M * K * 20, all = rows * kpad; // in twentieths
-    if (split_pw2_shape(d)) return real >= 14 * all;
-    if (real < (d->kh * d->kw > 1 ? 13 : 15) * all || c.groups_k < 3 || (M > 64 && 5 * K < 4 * kpad)) return false;
-    if (c.bm == 128) return true;
+    const int64_t real = (int64_t)M * K, all = rows * kpad;
+    // The last round: two workgroups that share a CU take 2000 cycles a slice, one alone 1700.
+    // Where whole 128-row tiles lose half of their rate to it and to padding, a little over one
+    // or two tiles per CU, the smaller fp32 tiles are faster (32 -> 432 3x3 stride 2, 284 tiles:
+    // 1.30; 280 -> 1824@21x21 with a residual, 525: 1.26; 624 -> 448@46x46, 268: 1.09).
+    const int64_t t128 = rows / 128 * ((ntot + 63) / 64) * d->group;
+    if (c.bm == 128 && !c.sk && t128 > cus) {
+        const int64_t rem = t128 % (2 * cus);
+        const int64_t cycles = t128 / (2 * cus) * 2000 + (rem == 0 ? 0 : rem <= cus ? 1700 : 2000);
+        if (1000. * t128 / ((double)cycles * cus) * real < 0.5 * all) return false;
+    }
+    if (split_pw2_shape(d)) return 20 * real >= 14 * all;
+    const int least = d->kh * d->kw == 1 ? 15 : M > 64 ? 14 : 13; // twentieths
+    if (20 * real < least * all || c.groups_k < 3 || (M > 64 && 5 * K < 4 * kpad)) return false;
+    // Channel tails pay from one and a half 64-row tiles per CU (614 -> 376, 216 tiles: 1.30).
+    if (d->c / d->group % 8 != 0 && 2 * tiles64 < 3 * cus) return false;
     // 64-row tiles, two to a CU, with 1-pixel loads: a little over one per CU, or two to three,
     // leave most of the last round empty, where smaller fp32 tiles do not (112 -> 192 3x3
-    // stride 2, 273 tiles: 1.11; 176 -> 64, 601 tiles: 1.13); channel tails pay from one and
-    // a half per CU (614 -> 376, 216 tiles: 1.30).
-    if ((tiles64 > cus && 4 * tiles64 < 5 * cus) || (tiles64 > 2 * cus && tiles64 < 3 * cus)) return false;
-    return d->c / d->group % 8 == 0 || 2 * tiles64 >= 3 * cus;
+    // stride 2, 273 tiles: 1.11; 176 -> 64, 601 tiles: 1.13); under one per CU the fp32 tiles
+    // split a K of 1536 and more (464 -> 152 3x3 stride 2, 192 tiles: 75 -> 93).
+    if (c.bm == 64 && tiles64 < cus && K >= 1536) return false;
+    return c.bm == 128 || !((tiles64 > cus && 4 * tiles64 < 5 * cus) || (tiles64 > 2 * cus && tiles64 < 3 * cus));
 }
 
 int64_t split_packed_floats(const SpinnHipConvDesc *d) {

@@ -285,8 +285,10 @@ def test_conv_uses_bf16_parts(native):
     assert parts(16, 96, 40, 256) and not parts(16, 72, 40, 256)      # K = 96 and 72 of 128
     assert parts(16, 192, 41, 256) and not parts(16, 136, 41, 256)    # K = 192 and 136 of 192, 1-pixel loads
     # 64-row tiles with 1-pixel loads: 211 and 500 of them, not 263 or 605
-    assert parts(16, 176, 57, 64, 3, 2) and parts(38, 176, 57, 64, 3, 2)
-    assert not parts(20, 176, 57, 64, 3, 2) and not parts(46, 176, 57, 64, 3, 2)
+    assert parts(16, 160, 57, 64, 3, 2) and parts(38, 160, 57, 64, 3, 2)
+    assert not parts(20, 160, 57, 64, 3, 2) and not parts(46, 160, 57, 64, 3, 2)
+    assert not parts(16, 176, 57, 64, 3, 2)        # K = 1584 under one tile per CU
+    assert not parts(14, 32, 36, 432, 3, 2)        # 284 128-row tiles, a little over one per CU
     assert not parts(16, 614, 29, 64) and parts(30, 614, 29, 64)      # a channel tail: 211, 395
     assert not parts(4, 16, 83, 304, 3)            # K = 144 of 192
     d = native.ConvDesc(1, 6, 8, 8, 4, 8, 8, 3, 3, 1, 1, 1, 1, 4, 0, 0, 0)
@@ -307,7 +309,7 @@ def test_wavek_switch_covers_every_conv(native):
 import ctypes as C
 from spinn_amd import native
 L = native.lib()
-for n, c, h, oc, k, s in ((32, 2048, 7, 512, 1, 1), (32, 1024, 14, 256, 1, 1), (32, 256, 28, 256, 3, 2)):
+for n, c, h, oc, k, s in ((32, 2048, 7, 512, 1, 1), (32, 256, 14, 1024, 1, 1), (32, 512, 14, 512, 3, 2)):
     o = (h - 1) // s + 1
     d = native.ConvDesc(n, c, h, h, oc, o, o, k, k, s, s, k // 2, k // 2, 1, 0, native.ALGO_IMPLICIT_GEMM, 0)
     print(L.spinn_hip_conv_workspace_size(C.byref(d)))
