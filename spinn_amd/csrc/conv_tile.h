@@ -1,7 +1,6 @@
-// conv_tile.h - an implicit-GEMM conv output tile: arguments, accumulator start and store.
-//
-// Shared by the kernels whose waves hold 32x32 accumulator blocks (conv_igemm.hip,
-// conv_split.hip).
+// conv_tile.h - an implicit-GEMM conv launch's arguments and its split-K reduction (the
+// fp32 tiles of conv_igemm.hip and the split-bf16 ones of conv_split.h), and the accumulator
+// start and store of waves that hold 32x32 blocks (conv_igemm.hip).
 #pragma once
 #include "mfma_core.h"
 #include "spinn_hip_internal.h"

@@ -12,8 +12,8 @@
 //     workgroup, one extra workgroup per CU; a range may end one tile and
 //     start the next. Extra workgroups have the lowest block ids, so they are
 //     dispatched, and their parts finished, first.
-//   PARTS_IN_DP (otherwise): each remaining tile in p equal parts of >= 4
-//     slices, one part done by each of the first R*p data-parallel workgroups
+//   PARTS_IN_DP (otherwise): each remaining tile in p equal parts of at least
+//     plan_streamk's min_part slices, one part done by each of the first R*p data-parallel workgroups
 //     before its own tile, so no workgroup beyond one per slot is launched.
 // The dispatcher deals workgroups to the 8 XCDs round-robin: each XCD gets a
 // contiguous run of whole tiles and its own share of the remaining ones, so
@@ -123,7 +123,7 @@ __device__ __forceinline__ bool sk_arrive(const SkSched &s, int cnt_idx, int npa
 // and loads marked sc0 suffice. Correctness there does not rest on sc0 alone
 // (the compiler's memory model counts sc0 as workgroup scope, which may hit in
 // the CU's L1) but on no L1 holding a line of a part slot when the last part
-// reads it: every L1 is invalidated when a launch starts, slots are 64x64x4 B
+// reads it: every L1 is invalidated when a launch starts, slots are whole tiles (16 KB and more)
 // (whole cache lines, one slot per part), and within a launch each slot's lines
 // are read once, by the tile's last part, after every part's stores completed
 // (s_waitcnt before the arrival); the only earlier access from any CU is the
@@ -198,11 +198,14 @@ __device__ __forceinline__ bool sk_finish_part(const SkSched &s, int nslots, int
     return true;
 }
 
-// The schedule of one workgroup. segment(t, k0, k1, acc) computes K slices [k0, k1) of
+// The schedule of one workgroup. SPLIT_WGS: block ids below 8 * s.W run a range of at most
+// S slices of the remaining tiles (the end of one tile and the start of the next), the rest
+// one whole tile each. PARTS_IN_DP: every block runs one whole tile, the first R * p of them
+// a part of a remaining tile before it. segment(t, k0, k1, acc) computes K slices [k0, k1) of
 // tile t (starting from the epilogue's terms when k0 == 0) and ends with every wave past
-// its last LDS read of the K loop; store(t, acc) applies the post-op and stores. Segments
-// are unrolled: a loop would keep the second segment's set-up live across the first's K
-// loop.
+// its last LDS read of the K loop; store(t, acc) applies the post-op and stores the segment
+// just computed or summed. Segments are unrolled: a loop would keep the second segment's
+// set-up live across the first's K loop and cost a wave per SIMD.
 template <int SCHEME, int NA, int TILE, class Acc, class Segment, class Store>
 __device__ __forceinline__ void sk_run(const SkSched &s, int tid, int &flag, const Segment &segment,
                                        const Store &store) {
