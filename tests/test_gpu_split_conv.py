@@ -2,9 +2,10 @@
 
 Forced onto shapes at the edges of its tiles and loaders and compared with a float64
 convolution. Bound: an operand's three parts are exact, the products left out stay below
-2^-25 of theirs, and the sum is rounded once per 32 k, so the relative L2 error stays below
+2^-24 of theirs, and the sum is rounded once per 32 k, so the relative L2 error stays below
 2^-24 (2 + sqrt(K / 32)); twice that is allowed. Inputs that bf16 parts cannot carry
-(infinities, NaN, magnitudes that round to infinity) must give what fp32 arithmetic gives.
+(infinities, NaN, magnitudes that round to infinity or lose bits) must give what fp32
+arithmetic gives.
 """
 import ctypes as C
 import math
@@ -69,7 +70,7 @@ def _exact(torch, shape, x, wt, b, r):
 def test_split_conv(hip, torch_gpu, tune, shape, bm, split, streamk):
     torch = torch_gpu
     n, c, h, w, oc, k, s, p, g, act = shape
-    if streamk == 1 and g == 1:  # more than a tile per CU, the remainder cut along K
+    if streamk == 1 and g == 1:  # more than a tile per CU (test_split_conv_streamk: real cuts)
         tune(1, bm, split)
         hip.lib().spinn_hip_tune_streamk(streamk)
         n = 256 * 64 // (((h + 2 * p - k) // s + 1) * ((w + 2 * p - k) // s + 1) * ((oc + 63) // 64))
@@ -205,3 +206,96 @@ def test_split_conv_tiny_sums_of_one_row(hip, torch_gpu, tune, row, hw, bm):
     y, _ = run_conv(hip, torch_gpu, d, x, wt)
     ref = x[:, 9].astype(np.float64) * 1.5
     assert (np.abs(y[:, row] - ref) <= 2.0 ** -149).all()
+
+
+# (n, c, h, w, oc, k, stride, pad, group, act), tile rows: what the cut is
+STREAMK = [
+    ((64, 256, 14, 14, 128, 1, 1, 0, 1, 1), 64),    # 392 tiles of 4 groups: extra workgroups
+    ((64, 256, 14, 14, 256, 1, 1, 0, 1, 5), 128),   # the same, 128 rows and a residual
+    ((136, 256, 14, 14, 128, 1, 1, 0, 1, 1), 64),   # 834: parts in whole-tile workgroups
+    ((32, 256, 14, 14, 1024, 1, 1, 0, 1, 5), 0),    # 784 128-row tiles, by the rule
+    ((64, 64, 14, 14, 128, 3, 1, 1, 1, 5), 64),     # 1-pixel loads, 9 groups
+    ((64, 64, 14, 14, 256, 3, 1, 1, 1, 0), 128),
+    ((64, 250, 14, 14, 128, 1, 1, 0, 1, 3), 64),    # a channel tail
+    ((64, 250, 14, 14, 256, 1, 1, 0, 1, 1), 128),
+]
+
+
+@pytest.mark.parametrize("special", [False, True], ids=["plain", "special"])
+@pytest.mark.parametrize("case", STREAMK, ids=[repr(c) for c in STREAMK])
+def test_split_conv_streamk(hip, torch_gpu, tune, case, special):
+    """Remaining tiles cut along K, each part starting inside it."""
+    shape, bm = case
+    n, c, h, w, oc, k, s, p, g, act = shape
+    print(f"[split conv stream-K] {case} special {special}", flush=True)
+    if bm:
+        tune(1, bm, 0)
+        hip.lib().spinn_hip_tune_streamk(1)
+    d = conv_desc(hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM)
+    assert hip.lib().spinn_hip_conv_uses_bf16_parts(C.byref(d)) == 1
+    ws = hip.lib().spinn_hip_conv_workspace_size(C.byref(d))
+    assert ws > 0 and ws % (4 * n * oc * h * w) != 0, "a K split's workspace holds whole outputs"
+    x, wt, b, r = _case(shape)
+    if special:
+        _plant(shape, x, wt, r)
+    y, _ = run_conv(hip, torch_gpu, d, x, wt, b, r)
+    _check(torch_gpu, shape, x, wt, b, r, y)
+
+
+def _plant(shape, x, wt, r):
+    """Infinities, NaN, values that round to infinity in bf16, tiny and subnormal ones."""
+    n, c, h, w = shape[:4]
+    ww = wt.reshape(wt.shape[0], -1)
+    x[0, 3, 2, 2], x[0, 5, 4, 3] = np.inf, np.nan
+    x[-1, 2, 5, 5], x[-1, 7, 0, 0], x[n // 2, c - 1, h - 1, w - 1] = 3.4e38, 1e-30, -np.inf
+    x[:, 1] *= np.float32(1e-3)
+    x[:, 4] *= np.float32(1e-36)
+    wt[1] *= np.float32(1e-6)
+    wt[3] *= np.float32(1e-36)
+    wt[5] *= np.float32(1e-42)
+    wt[7] *= np.float32(1e20)
+    wt[9] = 0
+    ww[2, 0], ww[4, ww.shape[1] - 1], ww[6, ww.shape[1] // 2] = np.inf, 3.4e38, np.nan
+    if r is not None:
+        r[0, 5, 1, 1] = np.inf
+
+
+def _check(torch, shape, x, wt, b, r, y):
+    """Every element against fp32 arithmetic: the same non-finite ones; finite ones within the
+    roundings of a sum of K terms in two-term steps, each at most 2^-24 of the terms' magnitudes
+    (and six products each off by fp32's least number). Sums near fp32's largest are skipped."""
+    n, c, h, w, oc, k, s, p, g, act = shape
+    kk = c // g * k * k
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref = _exact(torch, shape, x, wt, b, r)
+    ab = [None if a is None else np.abs(np.nan_to_num(a, nan=0.0, posinf=0.0, neginf=0.0)) for a in (x, wt, b, r)]
+    size = _exact(torch, shape[:9] + ((4,) if r is not None else (0,)), *ab)
+    fits = size < 1e38
+    assert fits.mean() > 0.5
+    nan = np.isnan(ref)
+    bad = np.argwhere((np.isnan(y) != nan) & (fits | nan))
+    assert len(bad) == 0, [(tuple(i), y[tuple(i)], ref[tuple(i)]) for i in bad[:8]]
+    inf = np.isinf(ref) & fits
+    assert np.array_equal(y[inf], ref[inf].astype(np.float32))
+    ok = np.isfinite(ref) & fits
+    assert ok.any()
+    err = np.abs(y[ok] - ref[ok])
+    lim = (kk / 2 + 8) * 2.0 ** -24 * size[ok] + 6 * kk * 2.0 ** -149
+    if act == 3:
+        lim = lim * 1.2 + 1e-6 * np.abs(ref[ok])  # silu's slope stays under 1.1; hardware exp2
+    worst = np.argmax(err - lim)
+    assert err[worst] <= lim[worst], (err[worst], lim[worst], y[ok][worst], ref[ok][worst])
+
+
+@pytest.mark.parametrize("bm,split", [(64, 1), (128, 1), (64, 3), (128, 2)])
+@pytest.mark.parametrize("shape", SHAPES, ids=[repr(s) for s in SHAPES])
+def test_split_conv_special_elements(hip, torch_gpu, tune, shape, bm, split):
+    """Special values on every loader, tile and K split, each element on its own."""
+    n, c, h, w, oc, k, s, p, g, act = shape
+    print(f"[split conv special] {shape} bm {bm} split {split}", flush=True)
+    tune(1, bm, split)
+    x, wt, b, r = _case(shape)
+    _plant(shape, x, wt, r)
+    d = conv_desc(hip, n, c, h, w, oc, k, k, s, s, p, p, g, act, hip.ALGO_IMPLICIT_GEMM)
+    y, _ = run_conv(hip, torch_gpu, d, x, wt, b, r)
+    _check(torch_gpu, shape, x, wt, b, r, y)
