@@ -432,7 +432,14 @@ __global__ __launch_bounds__(kThreads, 2) void conv_split_kernel(ConvSplitArgs a
     const int g1 = SPLIT ? min(a.groups_k, g0 + a.chunk) : a.groups_k;
     f32x4 acc[T::TM][T::TN];
     split_conv_segment<T, BL, RES>(a, group, m0, n0, g0, g1, !SPLIT, lds, lost, acc, tid, lane);
+    // Opaque copies (split_check): what the store shares with the prologue, above all the
+    // division of its columns, would stay in registers over the K loop, and a spilled index
+    // read back there waits for every load in flight (1-pixel loads, 128 rows, up to 12 %).
+    // The others do not spill, and computing it twice costs them 1-2 %.
+    int ln = lane, mw = m0, nw = n0;
+    if constexpr (T::BM == 128 && T::CW == 1) asm volatile("" : "+v"(ln), "+s"(mw), "+s"(nw));
     auto store = [&] {
+        const int lane = ln, m0 = mw, n0 = nw;
         if constexpr (SPLIT) {
             const int ntot = a.t.geom.ntot;
 #pragma unroll
@@ -475,12 +482,17 @@ __global__ __launch_bounds__(kThreads, 2) void conv_split_sk_kernel(ConvSplitArg
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     typedef f32x4 Acc[T::TM][T::TN];
     auto segment = [&](int t, int k0, int k1, Acc &acc) {
+        // Opaque copies, so that the segments share nothing over each other's K loops.
+        int ln = lane, td = tid;
+        if constexpr (T::BM == 128 && T::CW == 1) asm volatile("" : "+v"(ln), "+v"(td));
         const int m0 = (t % s.tiles_m) * T::BM + wave * T::WM, n0 = (t / s.tiles_m) * kSplitBN;
-        split_conv_segment<T, BL, RES>(a, 0, m0, n0, k0, k1, k0 == 0, lds, lost, acc, tid, lane);
-        split_check<T, RES>(a, 0, m0, n0, k0, k1, k0 == 0, acc, lost, lane, [] {});
+        split_conv_segment<T, BL, RES>(a, 0, m0, n0, k0, k1, k0 == 0, lds, lost, acc, td, ln);
+        split_check<T, RES>(a, 0, m0, n0, k0, k1, k0 == 0, acc, lost, ln, [] {});
     };
     auto store = [&](int t, const Acc &acc) {
-        split_store<T, AC>(a.t, 0, (t % s.tiles_m) * T::BM + wave * T::WM, (t / s.tiles_m) * kSplitBN, lane, acc);
+        int ln = lane; // opaque, as in conv_split_kernel
+        if constexpr (T::BM == 128 && T::CW == 1) asm volatile("" : "+v"(ln), "+s"(t));
+        split_store<T, AC>(a.t, 0, (t % s.tiles_m) * T::BM + wave * T::WM, (t / s.tiles_m) * kSplitBN, ln, acc);
     };
     sk_run<SCHEME, T::TM * T::TN * 4, T::BM * kSplitBN, Acc>(s, tid, sk_last, segment, store);
 }
