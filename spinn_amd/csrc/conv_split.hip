@@ -65,11 +65,11 @@ bool split_pw2_shape(const SpinnHipConvDesc *d) {
 // Tile height, K split and stream-K plan of an eligible conv. A 128-row tile splits each
 // activation half as often as a 64-row one and two workgroups share a CU, so it wins
 // where its grid has 0.6 of a tile per CU, two thirds with 1-pixel loads (320 -> 120 3x3
-// stride 2, 159 tiles: 115 against 91 on fp32 tiles) (MI355X, us: 512 -> 128@28x28 at batch 32, 392
-// tiles, 24.8 against 29.5 on 64 rows; 1024 -> 512@14x14 40.8 / 52.8; 3x3 stride 2
+// stride 2, 159 tiles: 115 us against 91 on fp32 tiles), unless M leaves over a fifth of its
+// rows empty (MI355X, us: 512 -> 128@28x28 at batch 32, 392 tiles, 24.8 against 29.5 on 64 rows; 1024 -> 512@14x14 40.8 / 52.8; 3x3 stride 2
 // 128@56x56 59.3 / 81.6; 256 -> 1024@14x14 at batch 8, 208 tiles, 10.1 / 11.2; 3x3 stride 2
 // 256@28x28 at batch 32, 196 tiles, 68.8 / 81.6, 76.0 with the remainder of the 64-row tiles
-// cut along K), unless M leaves over a fifth of its rows empty. One exception: 1x1 convs of
+// cut along K). One exception: 1x1 convs of
 // 2-pixel loads with 0.6 to 1 tile per CU and K of 768 or more run on 64 rows with the
 // remainder cut, though whole 128-row tiles are faster (1024 -> 256@14x14 at batch 32: 29.8
 // against 26.6): the tests of the workspace and no-allocation interfaces are written on this
@@ -80,7 +80,9 @@ bool split_pw2_shape(const SpinnHipConvDesc *d) {
 //  * else 64 rows, whole.
 // With three or more whole tiles per CU the remainder is cut along K where whole tiles
 // alone are unbalanced (plan_streamk); with fewer the co-resident workgroups even out
-// by themselves (512 -> 128@28x28: 33.8 cut, 24.8 whole).
+// by themselves (512 -> 128@28x28: 33.8 cut, 24.8 whole). Channel tails stay whole without a
+// residual: their cut kernel reads a spilled index back in its K loop (with one the other
+// does too: 359 -> 720@53x53 at batch 20 255 cut, 274 whole).
 SplitChoice split_choice(const SpinnHipConvDesc *d) {
     SplitChoice c{};
     const int M = d->oc / d->group;
@@ -93,6 +95,7 @@ SplitChoice split_choice(const SpinnHipConvDesc *d) {
     const int64_t t128 = (int64_t)((M + 127) / 128) * tiles_n * d->group;
     const bool fills = (M + 127) / 128 * 128 * 4 <= 5 * M;
     const bool pw2 = split_pw2_shape(d);
+    const bool res = d->act == SPINN_ACT_ADD || d->act == SPINN_ACT_ADD_RELU;
     const bool some = pw2 ? 5 * t128 >= 3 * cus : 3 * t128 >= 2 * cus;
     const bool cut = d->group == 1 && some && t128 < cus && c.groups_k >= 12 && pw2;
     int split = 1;
@@ -110,7 +113,7 @@ SplitChoice split_choice(const SpinnHipConvDesc *d) {
     if (d->group != 1) return c;
     if (const int k = g_force_split_k.load()) {
         split = k;
-    } else if (forced || (cut && c.bm == 64) || (c.bm == 128 && t128 >= 3 * cus)) {
+    } else if (forced || (cut && c.bm == 64) || (c.bm == 128 && t128 >= 3 * cus && (d->c % 8 == 0 || res))) {
         c.sk = plan_streamk((M + c.bm - 1) / c.bm, tiles_n, c.groups_k, 1, c.bm * kSplitBN, c.sp);
         if (c.sk) return c;
     }
@@ -131,6 +134,23 @@ bool split_eligible(const SpinnHipConvDesc *d) {
     // offsets stay inside the input. Planes are 1.5 times the weights: where they pass what
     // one buffer descriptor spans, the fp32 kernels still run.
     return d->c / d->group >= 16 && !stem_mfma_eligible(d) && split_plane_bytes(d) <= kMaxOperandBytes;
+}
+
+// How the fp32 kernels would run the conv (conv_igemm.hip): whole tiles in one launch, at
+// least one per CU; the wave-K kernel on a grid of one 64 x 64 tile per CU and more; or else
+// (K cut by stream-K or a reduction, or few tiles).
+enum Fp32Route { kFp32Whole, kFp32WaveK, kFp32Other };
+Fp32Route fp32_route(const SpinnHipConvDesc *d, const TileChoice &tc) {
+    const int M = d->oc / d->group, K = d->c / d->group * d->kh * d->kw, ntot = d->n * d->oh * d->ow;
+    if ((int64_t)((M + 63) / 64) * ((ntot + 63) / 64) * d->group < device_cu_count()) return kFp32Other;
+    const bool pointwise = d->kh == 1 && d->kw == 1 && d->sh == 1 && d->sw == 1 && d->ph == 0 && d->pw == 0 &&
+                           d->oh == d->h && d->ow == d->w;
+    if (wavek_tile(M, ntot, K, d->group, pointwise ? kWkConvPointwise : kWkConvGather)) return kFp32WaveK;
+    const int tiles_m = (M + tc.bm - 1) / tc.bm, tiles_n = (ntot + tc.bn - 1) / tc.bn;
+    SkPlan sp;
+    if (tc.split > 1 || (d->group == 1 && plan_streamk(tiles_m, tiles_n, (K + kBK - 1) / kBK, 4, tc.bm * tc.bn, sp)))
+        return kFp32Other;
+    return kFp32Whole;
 }
 
 } // namespace
@@ -160,40 +180,41 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     const int64_t cus = device_cu_count();
     if ((M + 63) / 64 * 64 * 3 > 4 * M || K < (res ? 256 : 64)) return false;
     if (!(tiles64 >= cus || (3 * tiles64 >= 2 * cus && K >= 256))) return false;
-    // What the tiles do for padding counts against their rate: rows up to 64 or 128, and K up
-    // to whole groups of 64. Over 4000 shapes of 32-2048 channels, 7-112 pixels and batches of
-    // 1-32, against the kernels they had (fp32 tiles, split K, wave-K), at a real share of
-    //   under 0.7   0.93-1.19 of the time for 1x1 convs with 2-pixel loads, half of them
-    //               slower (96 -> 2016@16x16: K = 96 in two groups, 1.4), above it 0.79;
-    //   under 0.75  up to 1.47 for 1x1 convs with 1-pixel loads (64 -> 723@69x69 at batch 23:
-    //               167 -> 246), above it 0.84; 3x3 ones gain down to 0.65, past 64
-    //               rows to 0.7 (280 -> 88@55x55 at batch 17: 140 -> 173) and not with K under
-    //               four fifths of its groups (16 -> 304@83x83 at batch 4: 33 -> 40);
-    // and with 1-pixel loads one or two groups of K do not pay for their prologue (1.06).
+    // Both ways timed over 3400 such convs of 16-2048 channels, 7-112 pixels and batches of
+    // 1-32, on random operands. Where the fp32 kernels take whole tiles in one launch, what
+    // the tiles here do for padding (rows up to 64 or 128, K up to whole groups of 64) counts;
+    // where they cut K, by stream-K or a reduction, or run the wave-K kernel, this one gains
+    // also at a real share of a half (1x1: 0.70; 72 -> 1809@14x14 at batch 4: 14.5 -> 7.7).
     const SplitChoice c = split_choice(d);
-    const int64_t rows = (M + c.bm - 1) / c.bm * c.bm, kpad = (int64_t)c.groups_k * kSplitGS * kSplitBK;
-    const int64_t real = (int64_t)M * K, all = rows * kpad;
-    // The last round: two workgroups that share a CU take 2000 cycles a slice, one alone 1700.
-    // Where whole 128-row tiles lose half of their rate to it and to padding, a little over one
-    // or two tiles per CU, the smaller fp32 tiles are faster (32 -> 432 3x3 stride 2, 284 tiles:
-    // 1.30; 280 -> 1824@21x21 with a residual, 525: 1.26; 624 -> 448@46x46, 268: 1.09).
-    const int64_t t128 = rows / 128 * ((ntot + 63) / 64) * d->group;
-    if (c.bm == 128 && !c.sk && t128 > cus) {
-        const int64_t rem = t128 % (2 * cus);
-        const int64_t cycles = t128 / (2 * cus) * 2000 + (rem == 0 ? 0 : rem <= cus ? 1700 : 2000);
-        if (1000. * t128 / ((double)cycles * cus) * real < 0.5 * all) return false;
-    }
-    if (split_pw2_shape(d)) return 20 * real >= 14 * all;
-    const int least = d->kh * d->kw == 1 ? 15 : M > 64 ? 14 : 13; // twentieths
-    if (20 * real < least * all || c.groups_k < 3 || (M > 64 && 5 * K < 4 * kpad)) return false;
-    // Channel tails pay from one and a half 64-row tiles per CU (614 -> 376, 216 tiles: 1.30).
-    if (d->c / d->group % 8 != 0 && 2 * tiles64 < 3 * cus) return false;
-    // 64-row tiles, two to a CU, with 1-pixel loads: a little over one per CU, or two to three,
-    // leave most of the last round empty, where smaller fp32 tiles do not (112 -> 192 3x3
-    // stride 2, 273 tiles: 1.11; 176 -> 64, 601 tiles: 1.13); under one per CU the fp32 tiles
-    // split a K of 1536 and more (464 -> 152 3x3 stride 2, 192 tiles: 75 -> 93).
-    if (c.bm == 64 && tiles64 < cus && K >= 1536) return false;
-    return c.bm == 128 || !((tiles64 > cus && 4 * tiles64 < 5 * cus) || (tiles64 > 2 * cus && tiles64 < 3 * cus));
+    const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((ntot + 63) / 64) * d->group;
+    const int64_t rem = tiles % (2 * cus);
+    const bool half = rem > 0 && rem <= cus; // the last round leaves one workgroup or none on a CU
+    const bool tail = d->c / d->group % 8 != 0, pw2 = split_pw2_shape(d), one = d->kh * d->kw == 1;
+    const TileChoice tc = choose_tiles(M, ntot, K, d->group, d->group == 1);
+    const Fp32Route route = fp32_route(d, tc);
+    // One fp32 chain over a long K would be nearly three times as far off (K = 2007, 954 tiles:
+    // 9.3e-7 against 3.3e-7): such layers stay here, also the slower ones (2007 -> 518@58x58 at
+    // batch 2, the worst: 134 -> 157).
+    if (route == kFp32Whole && K >= 1536) return true;
+    // 1x1 channel tails on 64-row tiles lose to all but the wave-K kernel (1527 -> 288, 285
+    // tiles: 1.17 of the time; half-empty last rounds 1.17, others 0.99).
+    if (c.bm == 64 && tail && one && route != kFp32WaveK) return false;
+    if (route != kFp32Whole) return true;
+    // The line by real share, in twentieths. Medians of the time (2-pixel loads; 1-pixel 1x1; larger
+    // kernels; channel tails): 0.5-0.6 1.14 / 1.14 / - / 1.26; 0.6-0.7 0.98 / 1.11 / 0.93 / 1.12;
+    // 0.7-0.8 0.87 / 0.96 / 0.82 / 0.82; above 0.74 / 0.80 / 0.71 / 0.78. Tails of 1x1 convs
+    // 1.03 at 0.7-0.8, above it 0.86.
+    const int64_t kpad = (int64_t)c.groups_k * kSplitGS * kSplitBK;
+    const int64_t real = 20 * (int64_t)M * K, all = (M + c.bm - 1) / c.bm * c.bm * kpad;
+    if (real < (pw2 || !one ? 13 : tail ? 16 : 14) * all) return false;
+    if (pw2) return true;
+    // 1x1 with 1-pixel loads: up to three groups of K do not pay for the prologue on 64-row
+    // tiles (1.04-1.35 of the time, four and more 0.87), nor up to two on 128-row ones in a
+    // half-empty last round or with a channel tail (1.00-1.05; three and more 0.77). Larger
+    // kernels: 16 channels into more than 64 do not (K = 144 of 192; 16 -> 304@83x83 at batch 4:
+    // 33 -> 40).
+    if (one && c.groups_k < (c.bm == 64 ? 4 : half || tail ? 3 : 1)) return false;
+    return one || M <= 64 || 5 * K >= 4 * kpad;
 }
 
 int64_t split_packed_floats(const SpinnHipConvDesc *d) {

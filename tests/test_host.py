@@ -281,16 +281,15 @@ def test_conv_uses_bf16_parts(native):
     assert not parts(32, 256, 28, 256, 3)          # Winograd
     assert parts(32, 256, 28, 256, 3, algo=native.ALGO_IMPLICIT_GEMM)
     assert not parts(32, 3, 224, 64, 7, 2)         # stem
-    assert parts(16, 64, 56, 256) and not parts(16, 64, 57, 256)      # one group of K: 2-pixel loads only
-    assert parts(16, 96, 40, 256) and not parts(16, 72, 40, 256)      # K = 96 and 72 of 128
-    assert parts(16, 192, 41, 256) and not parts(16, 136, 41, 256)    # K = 192 and 136 of 192, 1-pixel loads
-    # 64-row tiles with 1-pixel loads: 211 and 500 of them, not 263 or 605
-    assert parts(16, 160, 57, 64, 3, 2) and parts(38, 160, 57, 64, 3, 2)
-    assert not parts(20, 160, 57, 64, 3, 2) and not parts(46, 160, 57, 64, 3, 2)
-    assert not parts(16, 176, 57, 64, 3, 2)        # K = 1584 under one tile per CU
-    assert not parts(14, 32, 36, 432, 3, 2)        # 284 128-row tiles, a little over one per CU
-    assert not parts(16, 614, 29, 64) and parts(30, 614, 29, 64)      # a channel tail: 211, 395
-    assert not parts(4, 16, 83, 304, 3)            # K = 144 of 192
+    # fp32 alternatives of whole tiles: the share of the tiles that is real
+    assert parts(32, 64, 56, 256) and parts(32, 104, 56, 256) and not parts(32, 72, 56, 256)  # K of 64, 128, 128
+    assert parts(32, 136, 57, 256) and not parts(32, 136, 57, 240)        # K = 136 of 192, 1-pixel loads
+    assert not parts(32, 16, 111, 128, 3, 2)                              # K = 144 of 192
+    # fp32 alternatives that cut K or run the wave-K kernel: also at half a share
+    assert parts(4, 72, 14, 1808) and parts(9, 72, 28, 184)
+    # ... but not 1x1 channel tails on 64-row tiles
+    assert not parts(20, 614, 29, 64) and parts(20, 616, 29, 64)
+    assert parts(2, 2007, 58, 518)                                        # a long K: the smaller error
     d = native.ConvDesc(1, 6, 8, 8, 4, 8, 8, 3, 3, 1, 1, 1, 1, 4, 0, 0, 0)
     assert L.spinn_hip_conv_uses_bf16_parts(C.byref(d)) == 0          # refused
 
